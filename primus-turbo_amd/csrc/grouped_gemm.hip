@@ -8,6 +8,7 @@
 // no rows writes a zero slice.
 // Semantics follow primus_turbo/pytorch/kernels/grouped_gemm/grouped_gemm_fp8_impl.py:
 // 817-901 and the tail zeroing of grouped_gemm_kernel.py:1276-1310.
+#include "byte_transpose.h"
 #include "gemm_kernel.h"
 
 namespace pta {
@@ -32,47 +33,37 @@ __global__ __launch_bounds__(256) void zero_tail_kernel(const int64_t *offs, int
 
 // y[c, poffs[g] + r] = x[offs[g] + r, c] for r < len_g, 0 for len_g <= r < plen_g:
 // the token (K) axis of each group is moved to a 128-aligned column range of a
-// K-contiguous operand.  grid: (ceil(C/64), ceil(Mp/64)), Mp = M_total + 128*G.
-__global__ __launch_bounds__(256) void segment_transpose_kernel(const uint8_t *x, int64_t M_total, int64_t C,
-                                                                const int64_t *offs, const int64_t *poffs,
-                                                                int64_t G, int64_t ldy, uint8_t *y) {
-    __shared__ uint8_t s[64][68];
-    const int64_t c0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const int64_t p0 = static_cast<int64_t>(blockIdx.y) * 64; // padded column block
-    const int64_t Mp = poffs[G];
-    if (p0 >= Mp) return;
-    const int t = threadIdx.x;
-    // gather: local padded column p0 + r -> source token row (or -1 for padding)
-    {
-        const int     r  = t >> 2, cc = (t & 3) * 16;
-        const int64_t p  = p0 + r;
-        int64_t       src = -1;
-        if (p < Mp) {
-            int64_t lo = 0, hi = G - 1; // last g with poffs[g] <= p
-            while (lo < hi) {
-                const int64_t mid = (lo + hi + 1) >> 1;
-                if (poffs[mid] <= p) lo = mid;
-                else hi = mid - 1;
-            }
-            const int64_t rr = p - poffs[lo];
-            if (rr < offs[lo + 1] - offs[lo]) src = offs[lo] + rr;
-        }
-        for (int j = 0; j < 16; ++j) {
-            const int64_t c = c0 + cc + j;
-            s[r][cc + j]    = (src >= 0 && c < C) ? x[src * C + c] : 0;
-        }
+// K-contiguous operand, so a 128-wide tile of padded columns belongs to one
+// group (byte_transpose.h moves it; bound by memory).  grid: (ceil(C/128), ldy/128).
+template <int W>
+__global__ __launch_bounds__(BT_NT) void segment_transpose_kernel(const uint8_t *x, int64_t C, const int64_t *offs,
+                                                                  const int64_t *poffs, int64_t G, int64_t ldy,
+                                                                  uint8_t *y) {
+    static_assert(BT_TILE == 128, "a tile must not straddle two groups' 128-aligned ranges");
+    const int64_t c0 = static_cast<int64_t>(blockIdx.x) * BT_TILE;
+    const int64_t p0 = static_cast<int64_t>(blockIdx.y) * BT_TILE; // padded column block
+    if (p0 >= poffs[G]) return;
+    int64_t lo = 0, hi = G - 1; // last g with poffs[g] <= p0
+    while (lo < hi) {
+        const int64_t mid = (lo + hi + 1) >> 1;
+        if (poffs[mid] <= p0) lo = mid;
+        else hi = mid - 1;
     }
-    __syncthreads();
-    {
-        const int     r = t >> 2, cc = (t & 3) * 16; // r: output row (c), cc: column chunk
-        const int64_t c = c0 + r;
-        if (c < C) {
-            for (int j = 0; j < 16; ++j) {
-                const int64_t p = p0 + cc + j;
-                if (p < Mp) y[c * ldy + p] = s[cc + j][r];
-            }
-        }
-    }
+    const int64_t r0 = p0 - poffs[lo], left = offs[lo + 1] - offs[lo] - r0;
+    const int     rows = static_cast<int>(left < 0 ? 0 : (left < BT_TILE ? left : BT_TILE));
+    const int     cols = static_cast<int>(C - c0 < BT_TILE ? C - c0 : BT_TILE);
+    byte_transpose_tile<W>(x + (offs[lo] + r0) * C + c0, C, rows, cols, y + c0 * ldy + p0, ldy, BT_TILE);
+}
+
+int segment_transpose(const uint8_t *x, int64_t C, const int64_t *offs, const int64_t *poffs, int64_t G, int64_t ldy,
+                      uint8_t *y, hipStream_t st) {
+    const dim3 grid(static_cast<uint32_t>(cdiv(C, BT_TILE)), static_cast<uint32_t>(ldy / BT_TILE));
+    const int  ax = bt_access(x, C), ay = bt_access(y, ldy), w = ax < ay ? ax : ay;
+    if (w == 16) segment_transpose_kernel<16><<<grid, BT_NT, 0, st>>>(x, C, offs, poffs, G, ldy, y);
+    else if (w == 8) segment_transpose_kernel<8><<<grid, BT_NT, 0, st>>>(x, C, offs, poffs, G, ldy, y);
+    else segment_transpose_kernel<1><<<grid, BT_NT, 0, st>>>(x, C, offs, poffs, G, ldy, y);
+    PTA_CHECK_LAUNCH();
+    return PTA_OK;
 }
 
 int gran_sm(int gran) {
@@ -181,10 +172,14 @@ extern "C" int pta_grouped_gemm_fp8(const void *a, int a_fmt, const void *a_scal
     return PTA_OK;
 }
 
+// row stride of the transposed operands: room for every group's padding, whole
+// 128-column tiles
+static int64_t variable_k_pad(int64_t M_total, int64_t G) { return cdiv(M_total + 128 * G, 128) * 128; }
+
 extern "C" size_t pta_grouped_gemm_fp8_variable_k_workspace_size(int64_t M_total, int64_t OUT_M,
                                                                  int64_t OUT_N, int64_t G,
                                                                  int /*granularity*/) {
-    const int64_t Mp = M_total + 128 * G;
+    const int64_t Mp = variable_k_pad(M_total, G);
     return static_cast<size_t>(cdiv(Mp * OUT_M, 256) * 256 + cdiv(Mp * OUT_N, 256) * 256 +
                                cdiv((G + 1) * 8, 256) * 256);
 }
@@ -210,23 +205,15 @@ extern "C" int pta_grouped_gemm_fp8_variable_k(const void *lhs, int lhs_fmt, con
     const size_t  eb = c_dtype == PTA_F32 ? 4 : 2;
     const size_t  need = pta_grouped_gemm_fp8_variable_k_workspace_size(M_total, OUT_M, OUT_N, G, granularity);
     PTA_CHECK_ARG(workspace_bytes >= need && workspace, "workspace of %zu bytes required", need);
-    const int64_t Mp = M_total + 128 * G;
+    const int64_t Mp = variable_k_pad(M_total, G);
     uint8_t *lt = static_cast<uint8_t *>(workspace);
     uint8_t *rt = lt + cdiv(Mp * OUT_M, 256) * 256;
     int64_t *po = reinterpret_cast<int64_t *>(rt + cdiv(Mp * OUT_N, 256) * 256);
     // 128-aligned per-group column ranges (blockwise offsets are already aligned,
     // so for them this is a plain transpose)
     if (int rc = pta_grouped_compute_padded_offs(group_offs, po, G, 128, stream)) return rc;
-    {
-        const dim3 gl(static_cast<uint32_t>(cdiv(OUT_M, 64)), static_cast<uint32_t>(cdiv(Mp, 64)));
-        segment_transpose_kernel<<<gl, 256, 0, st>>>(static_cast<const uint8_t *>(lhs), M_total, OUT_M,
-                                                      group_offs, po, G, Mp, lt);
-        PTA_CHECK_LAUNCH();
-        const dim3 gr(static_cast<uint32_t>(cdiv(OUT_N, 64)), static_cast<uint32_t>(cdiv(Mp, 64)));
-        segment_transpose_kernel<<<gr, 256, 0, st>>>(static_cast<const uint8_t *>(rhs), M_total, OUT_N,
-                                                      group_offs, po, G, Mp, rt);
-        PTA_CHECK_LAUNCH();
-    }
+    if (int rc = segment_transpose(static_cast<const uint8_t *>(lhs), OUT_M, group_offs, po, G, Mp, lt, st)) return rc;
+    if (int rc = segment_transpose(static_cast<const uint8_t *>(rhs), OUT_N, group_offs, po, G, Mp, rt, st)) return rc;
     // NT problem per group: C[m, n] = sum_{k in seg} lhsT[m, k] rhsT[n, k]
     GemmArgs   g{};
     const bool swap = trans_c != 0; // C^T: exchange the operands

@@ -12,6 +12,7 @@
 // 304-460), which rules out saturating block maxima:
 //   E = floor(log2 amax) - emax_elem, plus 1 when amax * 2^-E > fp8_max,
 //   e8m0 = clamp(E + 127, 0, 254), q = fp8(x * 2^(127 - e8m0)).
+#include "byte_transpose.h"
 #include "common.h"
 
 #include <mutex>
@@ -937,34 +938,17 @@ template <int MODE> int launch_dequant(const DQArgs &a, int fmt, int out_dt, hip
 }
 
 // ---------------------------------------------------------------------------
-// byte transpose x[B, M, N] -> y[B, N, M], 64 x 64 tiles
+// byte transpose x[B, M, N] -> y[B, N, M], 128 x 128 tiles (byte_transpose.h;
+// MI355X, kernel trace: 14336 x 4096 22.7 us = 5.2 TB/s, 8192 x 14336 41.8 us =
+// 5.6 TB/s; 64 x 64 tiles moved byte by byte took 212 and 457 us)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void transpose_u8_kernel(const uint8_t *x, int64_t M, int64_t N, uint8_t *y) {
-    __shared__ uint8_t s[64][68];
-    const int64_t b = blockIdx.z, m0 = static_cast<int64_t>(blockIdx.y) * 64, n0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const uint8_t *xb = x + b * M * N;
-    uint8_t       *yb = y + b * M * N;
-    const int      t  = threadIdx.x;
-    // read: 64 rows x 64 bytes; lane t: row t>>2, 16 bytes at (t&3)*16
-    {
-        const int     r = t >> 2, c = (t & 3) * 16;
-        const int64_t m = m0 + r;
-        for (int j = 0; j < 16; ++j) {
-            const int64_t n = n0 + c + j;
-            s[r][c + j] = (m < M && n < N) ? xb[m * N + n] : 0;
-        }
-    }
-    __syncthreads();
-    {
-        const int     r = t >> 2, c = (t & 3) * 16; // r: output row (n), c: output col (m)
-        const int64_t n = n0 + r;
-        if (n < N) {
-            for (int j = 0; j < 16; ++j) {
-                const int64_t m = m0 + c + j;
-                if (m < M) yb[n * M + m] = s[c + j][r];
-            }
-        }
-    }
+template <int G>
+__global__ __launch_bounds__(BT_NT) void transpose_u8_kernel(const uint8_t *x, int64_t M, int64_t N, uint8_t *y) {
+    const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BT_TILE, n0 = static_cast<int64_t>(blockIdx.x) * BT_TILE;
+    const int64_t base = static_cast<int64_t>(blockIdx.z) * M * N;
+    const int     rows = static_cast<int>(M - m0 < BT_TILE ? M - m0 : BT_TILE);
+    const int     cols = static_cast<int>(N - n0 < BT_TILE ? N - n0 : BT_TILE);
+    byte_transpose_tile<G>(x + base + m0 * N + n0, N, rows, cols, y + base + n0 * M + m0, M, rows);
 }
 
 template <int IN_DT, int FMT>
@@ -1315,10 +1299,14 @@ extern "C" int pta_transpose_u8(const void *x, int64_t B, int64_t M, int64_t N, 
     clear_error();
     PTA_CHECK_ARG(x && y && B >= 1 && M >= 0 && N >= 0 && B <= 65535, "bad arguments");
     if (M == 0 || N == 0) return PTA_OK;
-    const dim3 grid(static_cast<uint32_t>(cdiv(N, 64)), static_cast<uint32_t>(cdiv(M, 64)),
-                    static_cast<uint32_t>(B));
-    transpose_u8_kernel<<<grid, NT, 0, as_stream(stream)>>>(static_cast<const uint8_t *>(x), M, N,
-                                                            static_cast<uint8_t *>(y));
+    const uint8_t *xp = static_cast<const uint8_t *>(x);
+    uint8_t       *yp = static_cast<uint8_t *>(y);
+    const dim3     grid(static_cast<uint32_t>(cdiv(N, BT_TILE)), static_cast<uint32_t>(cdiv(M, BT_TILE)),
+                        static_cast<uint32_t>(B));
+    const int      ax = bt_access(x, N), ay = bt_access(y, M), g = ax < ay ? ax : ay;
+    if (g == 16) transpose_u8_kernel<16><<<grid, BT_NT, 0, as_stream(stream)>>>(xp, M, N, yp);
+    else if (g == 8) transpose_u8_kernel<8><<<grid, BT_NT, 0, as_stream(stream)>>>(xp, M, N, yp);
+    else transpose_u8_kernel<1><<<grid, BT_NT, 0, as_stream(stream)>>>(xp, M, N, yp);
     PTA_CHECK_LAUNCH();
     return PTA_OK;
 }
