@@ -9,17 +9,18 @@
 // Other layouts (NN / TN / trans_c) are reduced to NT on the host side.
 //
 // Tiling: block tile BM x BN x 128 over WGM x WGN waves, wave tile 64 (M) x
-// 128 (N) = 4 x 8 MFMA sub-tiles.  The MFMA is issued "transposed": its first
+// 128 (N) = 4 x 8 MFMA sub-tiles, half of its rows and columns in either half of
+// the block tile (so that half tiles are consumed and refilled one by one).  The MFMA is issued "transposed": its first
 // operand is the B tile (rows n) and its second the A tile (rows m), so lane l
 // holds C[m = l%16][n = 4*(l/16) .. +3] of each 16 x 16 sub-tile: one A row per
 // lane (one A scale per sub-tile) and four consecutive n (8-byte bf16 stores).
 //
 // Operands go global -> LDS with buffer_load_dwordx4 ... lds (no staging
-// VGPRs), double-buffered; the 16-byte chunk index of each 128-byte tile row
-// is XOR-swizzled (chosen on the global side, since lane i of an LDS-DMA
+// VGPRs), double-buffered by half tiles; the 16-byte chunk index of each 128-byte
+// tile row is XOR-swizzled (chosen on the global side, since lane i of an LDS-DMA
 // always lands at M0 + 16 i) so the MFMA fragment reads are conflict free.
 // Blockwise: each K block's MFMA writes a fresh partial that is scaled into
-// the fp32 accumulator by VALU FMAs two MFMAs later, so the VALU work
+// the fp32 accumulator by VALU FMAs a few MFMAs later, so the VALU work
 // (4 FMAs per MFMA) overlaps the matrix pipe.
 #pragma once
 #include "common.h"
@@ -40,9 +41,9 @@ constexpr int TM = WTM / 16;                // 4 MFMA sub-tiles along M per wave
 constexpr int TILE_A_BYTES = BM * BK;
 
 // Per-tile-width layout.  A wave owns 64 x (BN / 2) of C = TM x TN sub-tiles.
-// LDS: two stages of (A tile, B tile), then one scale slot per stage holding
-// the per-column B scales (1-D x 1-D blockwise, fp32) or the four E8M0 bytes
-// of every A and B row (MX: A rows at +0, B rows at +BM*4).  The epilogue
+// LDS: two stages of (A tile, B tile), then a ring of four scale slots: the fp32
+// scales (blockwise) or the four E8M0 bytes (MX) of every A row (+0) and B row
+// (+BM*4) of a K block.  The epilogue
 // reuses the space to stage the C tile as 16-bit rows padded by 16 bytes, so
 // the per-lane 8-byte writes of 16 consecutive rows hit distinct banks.
 template <int BNT>
@@ -56,7 +57,7 @@ struct TileCfg {
     static constexpr int SBASE_      = 2 * STAGE_;
     static constexpr int EPITCH_     = BN_ * 2 + 16;
     static constexpr int EPI_BYTES   = BM * EPITCH_;
-    static constexpr int MAIN_BYTES  = SBASE_ + 2 * SSLOT_;
+    static constexpr int MAIN_BYTES  = SBASE_ + 4 * SSLOT_;
     static constexpr size_t SMEM     = EPI_BYTES > MAIN_BYTES ? EPI_BYTES : MAIN_BYTES;
 };
 
@@ -176,9 +177,9 @@ __device__ __forceinline__ v4i make_desc(const void *p, int64_t bytes) {
                __builtin_amdgcn_readfirstlane(n), 0x00020000};
 }
 
-// 16 bytes per lane from desc[voff + soff] into LDS at m0 + 16 * lane.  The
-// instruction is hidden from the compiler's wait-count tracking on purpose:
-// completion is awaited explicitly (vmcnt(0) before the stage barrier).
+// LDS-DMA: N bytes per lane from desc[voff + soff] into LDS at m0 + N * lane.  The
+// instructions are hidden from the compiler's wait-count tracking on purpose:
+// completion is awaited explicitly (wait_dma_and_barrier).
 __device__ __forceinline__ void dma16(uint32_t lds_addr, int voff, v4i desc, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
@@ -186,8 +187,6 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, int voff, v4i desc, int
                    "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory", "m0");
 }
-
-// 4 bytes per lane from desc[voff + soff] into LDS at m0 + 4 * lane
 __device__ __forceinline__ void dma4(uint32_t lds_addr, int voff, v4i desc, int soff) {
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                  :
@@ -196,14 +195,36 @@ __device__ __forceinline__ void dma4(uint32_t lds_addr, int voff, v4i desc, int 
                  : "memory", "m0");
 }
 
-__device__ __forceinline__ void wait_dma_and_barrier() {
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+// The same, nothing unless kb < nk (wave-uniform); two 1 KB pieces for dma16x2_if.
+// The skip is a scalar branch inside the asm: as a C++ branch it ends the
+// scheduling region, and the register allocator then spills 150-200 VGPRs.
+__device__ __forceinline__ void dma16x2_if(int kb, int nk, uint32_t lds_addr, int voff0, int voff1, v4i desc, int soff) {
+    const uint32_t l = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile("s_cmp_lt_i32 %0, %7\n\ts_cbranch_scc0 .Ldma%=\n\t"
+                 "s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %3, %5, %6 offen lds\n\t"
+                 "s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds\n.Ldma%=:"
+                 :
+                 : "s"(kb), "s"(l), "s"(l + 8 * BK), "v"(voff0),
+                   "v"(voff1), "s"(desc), "s"(__builtin_amdgcn_readfirstlane(soff)), "s"(nk)
+                 : "memory", "m0", "scc");
+}
+__device__ __forceinline__ void dma4_if(int kb, int nk, uint32_t lds_addr, int voff, v4i desc, int soff) {
+    asm volatile("s_cmp_lt_i32 %0, %5\n\ts_cbranch_scc0 .Ldma%=\n\t"
+                 "s_mov_b32 m0, %1\n\tbuffer_load_dword %2, %3, %4 offen lds\n.Ldma%=:"
+                 :
+                 : "s"(kb), "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(desc),
+                   "s"(__builtin_amdgcn_readfirstlane(soff)), "s"(nk)
+                 : "memory", "m0", "scc");
 }
 
-// the K step's barrier once this wave's LDS reads of the stage have returned
-// as well: after it no wave reads the stage, so the next DMAs may overwrite it
-__device__ __forceinline__ void wait_all_and_barrier() {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+// The workgroup's barrier once this wave's LDS reads have returned and all but its
+// newest LEFT DMAs have landed, or all of them unless kb < nk.
+template <int LEFT> __device__ __forceinline__ void wait_dma_and_barrier(int kb, int nk) {
+    asm volatile("s_cmp_lt_i32 %0, %2\n\ts_cbranch_scc1 .Lwait%=\n\ts_waitcnt vmcnt(0)\n"
+                 ".Lwait%=:\n\ts_waitcnt vmcnt(%1) lgkmcnt(0)\n\ts_barrier"
+                 :
+                 : "s"(kb), "n"(LEFT), "s"(nk)
+                 : "memory", "scc");
 }
 
 __device__ __forceinline__ int64_t uniform64(int64_t v) {
@@ -394,87 +415,82 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     const int nk = static_cast<int>((K + BK - 1) / BK);
 
     // ---- LDS-DMA addressing -----------------------------------------------------
-    // wave w loads rows [w*RPW, (w+1)*RPW) of each operand tile, 8 rows per
+    // A stage is four 16 KB items: rows 0-127 / 128-255 of the A tile (a0, a1) and
+    // of the B tile (b0, b1).  Each wave moves 16 rows of every item, 8 rows per
     // instruction; lane i fills LDS chunk i of that 1 KB span = row i/8,
     // physical chunk i%8, which holds logical chunk (i%8) ^ swz(row).
-    constexpr int RPW_A = BM / NWAVES, RPW_B = BN_ / NWAVES;
-    constexpr int DA = RPW_A / 8, DB = RPW_B / 8;
-    const v4i  dA = make_desc(A + m0 * g.lda, (min<int64_t>(M - m0, BM) - 1) * g.lda + K);
-    const v4i  dB = make_desc(B + n0 * g.ldb, (min<int64_t>(N - n0, BN_) - 1) * g.ldb + K);
-    const int  lr = lane >> 3, lp = lane & 7;
-    const int  ch = lp ^ lr;            // rows of one DMA are 8 apart: same swizzle
-    const int  rowA0 = wave * RPW_A + lr, rowB0 = wave * RPW_B + lr;
-    int vA[DA], vB[DB];
+    const int rowsA = static_cast<int>(min<int64_t>(M - m0, BM)), rowsB = static_cast<int>(min<int64_t>(N - n0, BN_));
+    v4i       dA[2], dB[2];
 #pragma unroll
-    for (int d = 0; d < DA; ++d) vA[d] = (rowA0 + 8 * d) * static_cast<int>(g.lda) + 16 * ch;
+    for (int h = 0; h < 2; ++h) {
+        const int ra = rowsA - 128 * h, rb = rowsB - 128 * h;
+        dA[h] = make_desc(A + (m0 + 128 * h) * g.lda, ra > 0 ? (min(ra, 128) - 1) * g.lda + K : 0);
+        dB[h] = make_desc(B + (n0 + 128 * h) * g.ldb, rb > 0 ? (min(rb, 128) - 1) * g.ldb + K : 0);
+    }
+    const int lr = lane >> 3, lp = lane & 7;
+    const int ch = lp ^ lr;            // rows of one DMA are 8 apart: same swizzle
+    int       vA[2], vB[2];
 #pragma unroll
-    for (int d = 0; d < DB; ++d) vB[d] = (rowB0 + 8 * d) * static_cast<int>(g.ldb) + 16 * ch;
-    const bool ktail = (K % BK) != 0;
-    // 1-D B scales: lane i of wave w < 4 stages column n0 + 64 w + i
-    const v4i dSB    = make_desc(SB, g.sb_bytes);
-    const int sbl_vo = static_cast<int>((n0 + 64 * (wave & 3) + lane) * g.sb_m) * 4;
-    // MX exponent rows (byte strides sa_m / sb_m, multiples of 4): wave w < 4
-    // stages A rows 64 w .. 64 w + 63 and B rows 64 w .. 64 w + 63
-    const v4i dMXA   = make_desc(g.sa, g.sa_bytes), dMXB = make_desc(SB, g.sb_bytes);
-    const int mx_voa = static_cast<int>((m0 + 64 * (wave & 3) + lane) * g.sa_m);
-    const int mx_vob = static_cast<int>((n0 + 64 * (wave & 3) + lane) * g.sb_m);
-    const int mx_ksa = static_cast<int>(g.sa_k), mx_ksb = static_cast<int>(g.sb_k); // bytes per K block
-    // Operand DMAs are issued by waves 0 .. NWAVES/2-1 only, each for its own
-    // rows and those of wave + NWAVES/2 (the other wave on its SIMD, as waves
-    // go round-robin over the 4 SIMDs).  The non-issuing wave of each SIMD
-    // starts its MFMAs right after its fragment reads and keeps the matrix
-    // pipe busy while its partner issues (3% faster than every wave issuing
-    // its own rows at the headline shape).
-    constexpr int HALF = NWAVES / 2;
-    const bool    dma_wave = __builtin_amdgcn_readfirstlane(wave) < HALF;
-    const int     pA = HALF * RPW_A * static_cast<int>(g.lda), pB = HALF * RPW_B * static_cast<int>(g.ldb);
-    auto issue = [&](int kb, int stage) {
-        const int      k0 = kb * BK;
-        const uint32_t la = lds0 + stage * STAGE_ + wave * RPW_A * BK;
-        const uint32_t lb = lds0 + stage * STAGE_ + TILE_A_BYTES + wave * RPW_B * BK;
-        // chunks past K (last block only) read out of range and land as zeros;
-        // the row offset stays in the per-lane offset so partial tiles are
-        // range-checked by the descriptor
-        const bool last = ktail && kb + 1 == nk;
-        const bool oob  = last && k0 + 16 * ch >= K;
-        if (dma_wave) {
-#pragma unroll
-            for (int d = 0; d < DA; ++d) {
-                dma16(la + d * 8 * BK, oob ? 0x7fffffff - 64 : vA[d], dA, k0);
-                dma16(la + HALF * RPW_A * BK + d * 8 * BK, oob ? 0x7fffffff - 64 : vA[d] + pA, dA, k0);
-            }
-#pragma unroll
-            for (int d = 0; d < DB; ++d) {
-                dma16(lb + d * 8 * BK, oob ? 0x7fffffff - 64 : vB[d], dB, k0);
-                dma16(lb + HALF * RPW_B * BK + d * 8 * BK, oob ? 0x7fffffff - 64 : vB[d] + pB, dB, k0);
-            }
-        }
-        if constexpr (SM == SM_BLOCK && !B2D) {
-            // waves 0..3 each stage 64 column scales of this K block
-            if (wave < BN_ / 64)
-                dma4(lds0 + SBASE_ + stage * SSLOT_ + wave * 256, sbl_vo,
-                     dSB, static_cast<int>((kb + kb_base) * g.sb_k) * 4);
-        } else if constexpr (SM == SM_MX) {
-            // one dword (four 32-K exponents) per row, staged by the operand
-            // DMA waves: 64 A rows and 64 B rows each (all eight waves staging
-            // one block each measured 8-10% slower: it puts a DMA back into
-            // the other wave of every SIMD).  The four DMA waves cover the
-            // B exponents of a 256-column tile exactly (slots 4-7).
-            static_assert(BN_ == 256, "MX exponent staging assumes four 64-row B slots");
-            if (dma_wave) {
-                dma4(lds0 + SBASE_ + stage * SSLOT_ + (wave & 3) * 256, mx_voa, dMXA,
-                     static_cast<int>(kb + kb_base) * mx_ksa);
-                dma4(lds0 + SBASE_ + stage * SSLOT_ + (4 + (wave & 3)) * 256, mx_vob, dMXB,
-                     static_cast<int>(kb + kb_base) * mx_ksb);
-            }
+    for (int d = 0; d < 2; ++d) {
+        vA[d] = (wave * 16 + 8 * d + lr) * static_cast<int>(g.lda) + 16 * ch;
+        vB[d] = (wave * 16 + 8 * d + lr) * static_cast<int>(g.ldb) + 16 * ch;
+    }
+    // chunks of the last K block that lie past K read out of range, as zeros
+    const int  ktail = (K % BK) != 0 ? nk - 1 : 0x7fffffff;
+    const bool koob  = (nk - 1) * BK + 16 * ch >= K;
+    // per-K-block scales (blockwise fp32, MX four E8M0 bytes): one dword per A row
+    // (waves 0-3, 64 rows each) and per B row (waves 4-7) into a ring of four slots
+    constexpr bool HAS_S = SM == SM_BLOCK || SM == SM_MX;
+    v4i            dS{};
+    int            vS = 0, ksS = 0;
+    if constexpr (HAS_S) {
+        constexpr int es = SM == SM_MX ? 1 : 4;
+        const bool    isA = wave < 4;
+        const int64_t r   = (isA ? m0 : n0) + 64 * (wave & 3) + lane;
+        dS  = isA ? make_desc(g.sa, g.sa_bytes) : make_desc(SB, g.sb_bytes);
+        vS  = static_cast<int>(((isA ? A2D : B2D) ? (r >> 7) : r) * (isA ? g.sa_m : g.sb_m)) * es;
+        ksS = static_cast<int>(isA ? g.sa_k : g.sb_k) * es;
+    }
+    // The part-th item of K block kb (part 0: a0 and the scales, 1: b0, 2: a1, 3:
+    // b1); nothing past the last block: skipped by the ping-pong loop and the
+    // persistent kernels, read out of range (a descriptor with no records; LDS gets
+    // zeros) by the other interleaved loops, which the skip makes 1-1.7% slower
+    // (MX 8192 x 28672 x 8192 1344 against 1367 us; grouped MX, persistent, 1020
+    // against 1004).
+    constexpr bool PINGPONG = SM == SM_TENSOR || SM == SM_ROW || (SM == SM_BLOCK && B2D);
+    constexpr bool SKIP     = PINGPONG || PERSIST;
+    auto           issue    = [&](int kb, int part) {
+        const int      k0 = kb * BK, h = part >> 1, ks = (kb + static_cast<int>(kb_base)) * ksS;
+        const uint32_t ls = lds0 + SBASE_ + (kb & 3) * SSLOT_ + wave * 256;
+        const uint32_t l  = lds0 + (kb & 1) * STAGE_ + (part & 1) * TILE_A_BYTES + h * 128 * BK + wave * 16 * BK;
+        const bool     oob = kb >= ktail && koob;
+        const int      v0  = oob ? 0x7fffffff - 64 : ((part & 1) ? vB[0] : vA[0]);
+        const int      v1  = oob ? 0x7fffffff - 64 : ((part & 1) ? vB[1] : vA[1]);
+        v4i            d   = (part & 1) ? dB[h] : dA[h];
+        if constexpr (SKIP) {
+            if (HAS_S && part == 0) dma4_if(kb, nk, ls, vS, dS, ks);
+            dma16x2_if(kb, nk, l, v0, v1, d, k0);
+        } else {
+            v4i ds = dS;
+            ds[2]  = kb < nk ? ds[2] : 0;
+            d[2]   = kb < nk ? d[2] : 0;
+            if (HAS_S && part == 0) dma4(ls, vS, ds, ks);
+            dma16(l, v0, d, k0);
+            dma16(l + 8 * BK, v1, d, k0);
         }
     };
 
     // ---- fragment addressing: rows base + 16 i + lane%16 share one swizzle --
     const int fr   = lane & 15;
     const int fg   = lane >> 4;
-    const int aoff0 = lds_off(wm * WTM + fr, fg), aoff1 = lds_off(wm * WTM + fr, 4 + fg);
-    const int boff0 = TILE_A_BYTES + lds_off(wn * WTN_ + fr, fg), boff1 = TILE_A_BYTES + lds_off(wn * WTN_ + fr, 4 + fg);
+    const int aoff0 = lds_off(wm * 32 + fr, fg), aoff1 = lds_off(wm * 32 + fr, 4 + fg);
+    const int boff0 = TILE_A_BYTES + lds_off(wn * 64 + fr, fg), boff1 = TILE_A_BYTES + lds_off(wn * 64 + fr, 4 + fg);
+    // sub-tile (j, i) of the wave: rows row_of(i) + fr, columns col_of(j) + 4 fg .. +
+    // 3: 32 rows of each a-half and 64 columns of each b-half
+    auto row_in_tile = [](int i) { return (i >> 1) * 128 + (i & 1) * 16; };
+    auto col_in_tile = [](int j) { return (j >> 2) * 128 + (j & 3) * 16; };
+    auto row_of      = [&](int i) { return row_in_tile(i) + wm * 32; };
+    auto col_of      = [&](int j) { return col_in_tile(j) + wn * 64; };
 
     v4f acc[TN_][TM];
 #pragma unroll
@@ -482,214 +498,235 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[j][i] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    const int64_t mw    = m0 + wm * WTM;   // first m of this wave
-    const int64_t nbase = n0 + wn * WTN_;   // first n of this wave
+    // ---- main loop --------------------------------------------------------------
+    // Two loops over the same LDS items; both keep the operand DMAs of about one
+    // and a half K blocks in flight (counted vmcnt waits, never a full drain) and
+    // spread their issue over the step: 8 per wave and K block, addressed by SGPRs
+    // and five VGPRs so that nothing spills.  Same K order and scaling
+    // order in both, so the same bits.  What bounds them now is power: the clock
+    // falls to 1.9-2.0 GHz, and a variant that issues no DMAs (wrong results) gains
+    // 16% of the time with 11% of the cycles.
+    // Measured (MI355X, medians of alternating runs in one process, us; "one stage"
+    // is the form with both operands of the next K block fetched at the step's
+    // start and drained at its end):
+    //                                    one stage   ping-pong   interleaved
+    //   tensorwise 8192^3                   370.6       363.4       367.1
+    //   tensorwise 4096 x 18432 x 7168      390.4       376.0       380.8
+    //   1x128 by 128x128, same shape        452.8       449.7       460.4
+    //   grouped, 65536 rows, 32x2048x7168   958.7       892.7       906.6
+    //   1x128 by 1x128, 18432x7168x4096     559.2       568.9       545.7
+    //   grouped variable K, 2048x7168      1238.2      1203.4      1143.7
+    //   MX 8192 x 28672 x 8192             1445.4      1392.7      1365.0
+    // (before the skip of the DMAs past the last block, worth another 0.5-1.5% to
+    // the ping-pong loop),
+    // so 1-D by 1-D scales and MX take the interleaved loop, the others ping-pong.
+    // a phase's barrier: this wave's LDS reads are back, and all but its newest 8
+    // item DMAs (and one of scales) have landed; all of them where the items that
+    // would follow (of K block kb) do not exist
+    auto wait_items = [&](int kb) { wait_dma_and_barrier<HAS_S ? 9 : 8>(kb, nk); };
+    if constexpr (PINGPONG) {
+        // Two waves share a SIMD (w and w + 4).  A K block is two phases, one per
+        // b-half: a load section (LDS reads of the phase's fragments, DMA issue)
+        // and a compute section (16 MFMAs), each ended by the workgroup's barrier.
+        // Waves 4-7 run one section behind, so on every SIMD one wave feeds the
+        // matrix pipe while the other loads.  Phase 0 of block k reads a0, a1, b0
+        // and refills b1 of block k + 1 (its slot was read one phase earlier);
+        // phase 1 reads b1 and refills the scales, a0, a1 and b0 of block k + 2.
+        // Blockwise: a partial is scaled into acc NP MFMAs later, between MFMAs:
+        // the FMAs of a wave fill the shadow of its own MFMAs (12 of 16 partials;
+        // the last 4 wait for the next load section).  All FMAs in the load section
+        // leave the matrix pipe idle for their whole length, since waiting MFMAs
+        // hold the VALU port: 3911 against 3302 cycles per K block.
+        if (nk > 0) {
+            constexpr int NP = 4;
+            v8i   af[TM], bf[4];
+            float sa_r[TM] = {}, sb_u[2] = {}, s_q[TM] = {};
+            v4f   p[NP] = {};
+            auto scale_in = [&](int h, int q) { // acc += partial of tile q (0-15) of b-half h, scaled
+                acc[h * 4 + (q >> 2)][q & 3] += p[q % NP] * s_q[q & 3];
+            };
+            issue(0, 0); issue(0, 2); issue(0, 1); issue(0, 3);
+            issue(1, 0); issue(1, 2); issue(1, 1);
+            wait_items(1);
+            const bool late = wave >= 4;
+            if (late) asm volatile("s_barrier" ::: "memory");
 
-    // ---- scale addressing (32-bit offsets, per-K-block soffset) -------------
-    const rsrc_t rSA = make_rsrc(g.sa, g.sa_bytes);
-    const rsrc_t rSB = make_rsrc(SB, g.sb_bytes);
-    int          sa_vo[TM];
-    int          sb_vo[TN_];
-    int          sb_uo = 0;
-    if constexpr (SM == SM_BLOCK || SM == SM_MX) {
-        const int es = SM == SM_MX ? 1 : 4;
+            for (int kb = 0; kb < nk; ++kb) {
+                const uint8_t *S  = smem + (kb & 1) * STAGE_;
+                const float   *SC = reinterpret_cast<const float *>(smem + SBASE_ + (kb & 3) * SSLOT_);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int64_t r = min<int64_t>(mw + 16 * i + fr, M - 1);
-            sa_vo[i]        = static_cast<int>((A2D ? (r >> 7) : r) * g.sa_m) * es;
-        }
-        if constexpr (SM == SM_MX) {
+                for (int h = 0; h < 2; ++h) {
+                    // ---- load section
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (h == 0) {
 #pragma unroll
-            for (int j = 0; j < TN_; ++j) sb_vo[j] = static_cast<int>(min<int64_t>(nbase + 16 * j + fr, N - 1) * g.sb_m);
-        } else if constexpr (B2D) {
-            sb_uo = static_cast<int>((nbase >> 7) * g.sb_m) * 4;
-        }
-    }
-    // scales of one K block (loaded one block ahead)
-    struct Scales {
-        float sa[TM];
-        float sb_u;
-    };
-    auto load_scales = [&](int kb, Scales &s) {
-        if constexpr (SM == SM_BLOCK) {
-            const int ka  = static_cast<int>((kb + kb_base) * g.sa_k) * 4;
-            const int kbb = static_cast<int>((kb + kb_base) * g.sb_k) * 4;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) s.sa[i] = bload_f32(rSA, sa_vo[i], ka);
-            if constexpr (B2D) s.sb_u = bload_f32(rSB, sb_uo, kbb);
-        }
-    };
-
-    // ---- prologue ---------------------------------------------------------
-    Scales sc_cur{}, sc_nxt{};
-    if (nk > 0) {
-        load_scales(0, sc_cur);
-        issue(0, 0);
-    }
-    wait_dma_and_barrier();
-
-    // blockwise pipeline state: partial buffers p[4]; the two tiles issued last
-    // in a K block are scaled at the start of the next one with that block's scales
-    v4f    p[4];
-    float  s_pend[4];
-    v4f    pend4[2];
-    float4 sbj_prev = make_float4(0.f, 0.f, 0.f, 0.f);
-    bool   have_pend = false;
-
-    for (int kb = 0; kb < nk; ++kb) {
-        const int cur = kb & 1;
-        if (kb + 1 < nk) load_scales(kb + 1, sc_nxt);
-        const uint8_t *S = smem + cur * STAGE_;
-        v8i            af[TM];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) af[i] = frag(S, aoff0 + i * 16 * BK, aoff1 + i * 16 * BK);
-        float s_i[TM];
-        if constexpr (SM == SM_BLOCK && B2D) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) s_i[i] = sc_cur.sa[i] * sc_cur.sb_u;
-        }
-        v8i bf = frag(S, boff0, boff1);
-        // the next stage's DMAs go out behind this step's first fragment reads
-        // (stage cur ^ 1 was last read before the previous step's barrier)
-        if (kb + 1 < nk) issue(kb + 1, cur ^ 1);
-        const float *SBL = reinterpret_cast<const float *>(smem + SBASE_ + cur * SSLOT_) + wn * WTN_ + 4 * fg;
-        int ea[TM], eb[TN_];
-        if constexpr (SM == SM_MX) {
-            const uint8_t *EX = smem + SBASE_ + cur * SSLOT_;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) ea[i] = EX[(wm * WTM + 16 * i + fr) * 4 + fg];
-#pragma unroll
-            for (int j = 0; j < TN_; ++j) eb[j] = EX[BM * 4 + (wn * WTN_ + 16 * j + fr) * 4 + fg];
-        }
-        // Step barrier.  EARLY_BAR: the last B fragment is read three fragments
-        // ahead, and the barrier goes before fragment TN_ - 2's MFMAs with this
-        // wave's reads of the stage complete, so the stage is free once every
-        // wave has passed it and the rest of the step's MFMAs overlap the wait
-        // (as fast as a barrier the compiler hoists above the last read's
-        // wait, and formally race-free).  The 1-D x 1-D loop keeps its barrier
-        // at the end of the step (the early form measured 7-11% slower there):
-        // the scheduler hoists it above the MFMAs of the last fragment, after
-        // that fragment's reads are issued; those reads return long before the
-        // next step's DMAs into this stage, which other waves issue after the
-        // remaining MFMAs and which take hundreds of cycles to arrive.
-        constexpr bool EARLY_BAR = !(SM == SM_BLOCK && !B2D);
-        static_assert(!EARLY_BAR || TN_ >= 4, "the early barrier reads the last B fragment three ahead");
-        v8i            blast = bf;
-#pragma unroll
-        for (int j = 0; j < TN_; ++j) {
-            if (EARLY_BAR && j == TN_ - 2) {
-                __builtin_amdgcn_sched_barrier(0);
-                wait_all_and_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            float4 sbj = make_float4(0.f, 0.f, 0.f, 0.f);
-            if constexpr (SM == SM_BLOCK && !B2D) sbj = *reinterpret_cast<const float4 *>(SBL + 16 * j);
-            v8i bn = bf;
-            if (j + 1 < TN_ - (EARLY_BAR ? 1 : 0)) bn = frag(S, boff0 + (j + 1) * 16 * BK, boff1 + (j + 1) * 16 * BK);
-            if (EARLY_BAR && j == TN_ - 4) blast = frag(S, boff0 + (TN_ - 1) * 16 * BK, boff1 + (TN_ - 1) * 16 * BK);
-            if (EARLY_BAR && j == TN_ - 2) bn = blast;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int tt = j * TM + i;
-                if constexpr (SM == SM_BLOCK) {
-                    p[tt & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        bf, af[i], v4f{0.f, 0.f, 0.f, 0.f}, FB, FA, 0, 0, 0, 0);
-                    // scale the tile issued two MFMAs earlier
-                    if constexpr (B2D) {
-                        if (tt >= 2) {
-                            const int q = tt - 2;
-                            acc[q / TM][q % TM] += p[q & 3] * s_i[q % TM];
-                        } else if (have_pend) {
-                            const int q = TN_ * TM - 2 + tt; // tiles 30, 31 of the previous block
-                            acc[q / TM][q % TM] += p[q & 3] * s_pend[q & 3];
+                        for (int i = 0; i < TM; ++i) {
+                            const int ro = row_in_tile(i) * BK;
+                            af[i] = frag(S, aoff0 + ro, aoff1 + ro);
                         }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int co = col_in_tile(4 * h + j) * BK;
+                        bf[j] = frag(S, boff0 + co, boff1 + co);
+                        if constexpr (SM == SM_BLOCK) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (j < 3) {
+                                scale_in(h ^ 1, 16 - NP + j);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (h == 0) {
+                        issue(kb + 1, 3);
                     } else {
-                        // 1-D B scales: the tile issued two MFMAs earlier, whose B
-                        // scales are this fragment's (i >= 2) or the previous
-                        // one's (i < 2); deferring it was 7% faster than scaling
-                        // each partial right behind its MFMA
-                        if (tt >= 2) {
-                            const int    q  = tt - 2, iq = q % TM;
-                            const float4 sq = q / TM == j ? sbj : sbj_prev;
-                            const float  sa = sc_cur.sa[iq];
-                            acc[q / TM][iq][0] += p[q & 3][0] * (sa * sq.x);
-                            acc[q / TM][iq][1] += p[q & 3][1] * (sa * sq.y);
-                            acc[q / TM][iq][2] += p[q & 3][2] * (sa * sq.z);
-                            acc[q / TM][iq][3] += p[q & 3][3] * (sa * sq.w);
-                        } else if (have_pend) {
-                            const int q = TN_ * TM - 2 + tt;
-                            acc[q / TM][q % TM] += p[q & 3] * pend4[tt];
+                        issue(kb + 2, 0); issue(kb + 2, 2); issue(kb + 2, 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (SM == SM_BLOCK) {
+                        scale_in(h ^ 1, 15);
+                        if (h == 0) {
+#pragma unroll
+                            for (int i = 0; i < TM; ++i) sa_r[i] = SC[row_of(i) + fr];
+                            sb_u[0] = SC[BM + col_of(0)];
+                            sb_u[1] = SC[BM + col_of(4)];
                         }
-                        // per MFMA: the MFMA, four VALU, (first MFMA of each B
-                        // fragment) the next fragment's LDS reads and its B
-                        // scales, four VALU (4% faster than the compiler's order)
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); // VALU
-                        if (i == 0) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0); // DS read
-                        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); // VALU
                     }
-                    if constexpr (B2D) {
-                        // instruction order per MFMA: the MFMA, two VALU, (first
-                        // MFMA of each B fragment) the next fragment's two LDS
-                        // reads, two VALU.  The compiler's own order clusters
-                        // the FMAs right behind the MFMA that feeds them and pads
-                        // the result hazard with s_nop; this one is 4% faster.
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0); // VALU
-                        if (i == 0 || (i == 2 && j == TN_ - 4)) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0); // DS read
-                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0); // VALU
+                    __builtin_amdgcn_sched_barrier(0);
+                    wait_items(kb + 1 + h);
+                    __builtin_amdgcn_sched_barrier(0);
+                    // ---- compute section
+                    if constexpr (SM == SM_BLOCK) {
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) s_q[i] = sa_r[i] * sb_u[h];
                     }
-                } else if constexpr (SM == SM_MX) {
-                    acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        bf, af[i], acc[j][i], FB, FA, 0, eb[j], 0, ea[i]);
-                } else {
-                    acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        bf, af[i], acc[j][i], FB, FA, 0, 0, 0, 0);
-                    // the next B fragment's LDS reads go behind the second MFMA
-                    // of each fragment (4% faster than the compiler's order; the
-                    // same pattern measured slower for MX)
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-                    if (i == 1) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0); // DS read
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        const int j = q >> 2, i = q & 3;
+                        if constexpr (SM == SM_BLOCK) {
+                            if (q >= NP) {
+                                scale_in(h, q - NP);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                            p[q % NP] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                                bf[j], af[i], v4f{0.f, 0.f, 0.f, 0.f}, FB, FA, 0, 0, 0, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                        } else {
+                            acc[h * 4 + j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                                bf[j], af[i], acc[h * 4 + j][i], FB, FA, 0, 0, 0, 0);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_barrier" ::: "memory");
                 }
             }
-            bf = bn;
-            sbj_prev = sbj;
-        }
-        if constexpr (SM == SM_BLOCK && B2D) {
+            if (!late) asm volatile("s_barrier" ::: "memory");
+            if constexpr (SM == SM_BLOCK) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) s_pend[q] = s_i[q % TM];
-            have_pend = true;
-        }
-        if constexpr (SM == SM_BLOCK && !B2D) {
-            // tiles 30, 31 (fragment 7, i = 2, 3) are scaled in the next step
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const float sa = sc_cur.sa[TM - 2 + u];
-                pend4[u] = v4f{sa * sbj_prev.x, sa * sbj_prev.y, sa * sbj_prev.z, sa * sbj_prev.w};
-            }
-            have_pend = true;
-        }
-        sc_cur = sc_nxt;
-        if constexpr (!EARLY_BAR) wait_dma_and_barrier();
-    }
-    if constexpr (SM == SM_BLOCK && B2D) {
-        if (have_pend) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int q = TN_ * TM - 2 + tt;
-                acc[q / TM][q % TM] += p[q & 3] * s_pend[q & 3];
+                for (int u = 0; u < NP; ++u) scale_in(1, 16 - NP + u);
             }
         }
-    }
-    if constexpr (SM == SM_BLOCK && !B2D) {
-        if (have_pend) {
+    } else {
+        // A K block is two phases (b-halves) of 16 MFMAs per wave, tiles q = 16 h +
+        // 4 j + i; both waves of a SIMD run the same phase and interleave their MFMAs
+        // with each other's VALU work.  The next B fragment is read one fragment
+        // ahead.  Before each phase's last fragment (j = 3) comes the workgroup's
+        // barrier: after it the next phase's first fragments are read (every af[i]
+        // right behind its last MFMA), and the slots that the phase read are
+        // refilled two K blocks ahead (phase 0: scales, a0, a1, b0; phase 1: b1).
+        // 1-D by 1-D: a partial is scaled into acc LAG MFMAs later (3: the MFMA's
+        // result is there without s_nop).
+        if (nk > 0) {
+            constexpr int LAG = 3;
+            v8i   af[TM], bf[2];
+            float sa_r[TM] = {};     // A scales of the K block
+            v4f   sb_r[2]  = {};     // B scales of a fragment
+            v4f   s_p[LAG + 1] = {}; // scales of the last partials
+            int   ea[TM] = {}, eb[2] = {};
+            v4f   p[4] = {};
+            auto  read_a = [&](int kb, int i) {
+                const uint8_t *S  = smem + (kb & 1) * STAGE_;
+                const int      ro = row_in_tile(i) * BK;
+                af[i] = frag(S, aoff0 + ro, aoff1 + ro);
+            };
+            auto read_b = [&](int kb, int h, int j) {
+                const uint8_t *S  = smem + (kb & 1) * STAGE_;
+                const uint8_t *SC = smem + SBASE_ + (kb & 3) * SSLOT_;
+                const int      co = col_in_tile(4 * h + j) * BK;
+                bf[j & 1] = frag(S, boff0 + co, boff1 + co);
+                if constexpr (SM == SM_BLOCK)
+                    sb_r[j & 1] = *reinterpret_cast<const v4f *>(SC + (BM + col_of(h * 4 + j) + 4 * fg) * 4);
+                else eb[j & 1] = SC[(BM + col_of(h * 4 + j) + fr) * 4 + fg];
+            };
+            auto read_s = [&](int kb) {
+                const uint8_t *SC = smem + SBASE_ + (kb & 3) * SSLOT_;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int q = TN_ * TM - 2 + tt;
-                acc[q / TM][q % TM] += p[q & 3] * pend4[tt];
+                for (int i = 0; i < TM; ++i) {
+                    if constexpr (SM == SM_BLOCK) sa_r[i] = reinterpret_cast<const float *>(SC)[row_of(i) + fr];
+                    else ea[i] = SC[(row_of(i) + fr) * 4 + fg];
+                }
+            };
+            issue(0, 0); issue(0, 2); issue(0, 1); issue(0, 3);
+            // block 0's scales, a0, a1 and b0 have landed (requesting block 1 behind this
+            // wait instead of ahead of it: 66.8 -> 64.7 us at 7168 x 2048 x 4096)
+            asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
+            issue(1, 0); issue(1, 2); issue(1, 1); issue(1, 3);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) read_a(0, i);
+            read_b(0, 0, 0);
+            read_s(0);
+
+            for (int kb = 0; kb < nk; ++kb) {
+#pragma unroll
+                for (int q = 0; q < 32; ++q) {
+                    const int h = q >> 4, j = (q >> 2) & 3, i = q & 3;
+                    if (i == 0 && j == 3) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        wait_items(kb + 1 + h);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (SM == SM_BLOCK) {
+                        p[q & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            bf[j & 1], af[i], v4f{0.f, 0.f, 0.f, 0.f}, FB, FA, 0, 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        const int w = (q + 32 - LAG) & 31;
+                        acc[w >> 2][w & 3] += p[w & 3] * s_p[w % (LAG + 1)];
+                        s_p[q % (LAG + 1)] = sa_r[i] * sb_r[j & 1];
+                    } else {
+                        acc[h * 4 + j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            bf[j & 1], af[i], acc[h * 4 + j][i], FB, FA, 0, eb[j & 1], 0, ea[i]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (i == 0) {
+                        if (j < 3) read_b(kb, h, j + 1);
+                        else if (h == 0) read_b(kb, 1, 0);
+                        else read_b(kb + 1, 0, 0);
+                    }
+                    if (h == 1 && j == 3) {
+                        read_a(kb + 1, i);
+                        if (i == 3) read_s(kb + 1);
+                    }
+                    if (i == 1) {
+                        if (h == 0 && j == 3) issue(kb + 2, 0);
+                        if (h == 1 && j == 0) issue(kb + 2, 2);
+                        if (h == 1 && j == 1) issue(kb + 2, 1);
+                        if (h == 1 && j == 3) issue(kb + 2, 3);
+                    }
+                }
+            }
+            if constexpr (SM == SM_BLOCK) {
+#pragma unroll
+                for (int u = 0; u < LAG; ++u) {
+                    const int w = 32 - LAG + u;
+                    acc[w >> 2][w & 3] += p[w & 3] * s_p[w % (LAG + 1)];
+                }
             }
         }
     }
+    // DMAs past the last K block still write zeros to LDS
+    if constexpr (!SKIP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // ---- K split: the first half hands its accumulators to the second -------
     if constexpr (!PERSIST) {
@@ -765,16 +802,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 era[i] = 1.0f;
-                if constexpr (SM == SM_ROW) era[i] = reinterpret_cast<const float *>(g.sa)[mw + 16 * i + fr];
+                if constexpr (SM == SM_ROW) era[i] = reinterpret_cast<const float *>(g.sa)[m0 + row_of(i) + fr];
             }
-            // all waves are past their last fragment reads
+            // all waves are past their last fragment reads (and no DMA is in flight)
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
             for (int j = 0; j < TN_; ++j) {
                 float erb[4] = {1.f, 1.f, 1.f, 1.f};
                 if constexpr (SM == SM_ROW) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) erb[r] = reinterpret_cast<const float *>(SB)[nbase + 16 * j + 4 * fg + r];
+                    for (int r = 0; r < 4; ++r) erb[r] = reinterpret_cast<const float *>(SB)[n0 + col_of(j) + 4 * fg + r];
                 }
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
@@ -796,7 +833,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
                         lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((ef2{x[0], x[1]}), eh2));
                         hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((ef2{x[2], x[3]}), eh2));
                     }
-                    const int off = (wm * WTM + 16 * i + fr) * EPITCH_ + (wn * WTN_ + 16 * j + 4 * fg) * 2;
+                    const int off = (row_of(i) + fr) * EPITCH_ + (col_of(j) + 4 * fg) * 2;
                     *reinterpret_cast<uint2 *>(smem + off) = make_uint2(lo, hi);
                 }
             }
@@ -824,11 +861,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     float rs_a[TM];
     if constexpr (SM == SM_ROW) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) rs_a[i] = reinterpret_cast<const float *>(g.sa)[min<int64_t>(mw + 16 * i + fr, M - 1)];
+        for (int i = 0; i < TM; ++i) rs_a[i] = reinterpret_cast<const float *>(g.sa)[min<int64_t>(m0 + row_of(i) + fr, M - 1)];
     }
 #pragma unroll
     for (int j = 0; j < TN_; ++j) {
-        const int64_t n = nbase + 16 * j + 4 * fg;
+        const int64_t n = n0 + col_of(j) + 4 * fg;
         float         rs_b[4] = {1.f, 1.f, 1.f, 1.f};
         if constexpr (SM == SM_ROW) {
 #pragma unroll
@@ -836,7 +873,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const int64_t m = mw + 16 * i + fr;
+            const int64_t m = m0 + row_of(i) + fr;
             if (m >= M || n >= N) continue;
             float x[4];
 #pragma unroll
