@@ -122,6 +122,19 @@ int pta_quantize_fp8_rowwise(const void *x, int in_dtype, int64_t outer, int64_t
                              int64_t inner, const float *scale, void *q, int fmt, float *scale_inv,
                              void *workspace, size_t workspace_bytes, pta_stream_t stream);
 
+/* ROWWISE quantization of a matrix x[M, N] along its rows' axis (one scale per
+ * column), bytes written transposed: q_t[N, M], scale_inv[N].  M and N are
+ * multiples of 16, buffers 16-byte aligned.  With src_scale (one fp32 per row) x
+ * holds fp8 bytes of src_fmt, and an element enters as in_dtype(float(x) *
+ * src_scale[row]): the re-quantization of a rowwise-quantized tensor along its
+ * other axis without the dequantized copy.  workspace:
+ * pta_quantize_fp8_rowwise_workspace_size(1, M, N) bytes.  No counterpart in the
+ * reference, whose rowwise layer (ops/gemm_fp8.py:231-379) dequantizes,
+ * quantizes and transposes in separate calls. */
+int pta_quantize_fp8_rowwise_cols_t(const void *x, int in_dtype, int src_fmt, const float *src_scale, int64_t M,
+                                    int64_t N, void *q_t, int fmt, float *scale_inv, void *workspace,
+                                    size_t workspace_bytes, pta_stream_t stream);
+
 /* Blockwise 1-D: axis 1 -> 1 x block along N, s[M, ceil(N/block)];
  * axis 0 -> block x 1 along M, s[ceil(M/block), N]; eps 1e-4.
  * Replaces quant_fp8_blockwise_impl

@@ -476,23 +476,155 @@ __global__ __launch_bounds__(NT) void rw_col_partial_kernel(const void *x, int64
     partial[(o * nchunk + c) * inner + n] = a;
 }
 
+// 64 columns per workgroup, the chunks split over its 4 waves (one thread per
+// column walking all chunks took 31-54 us for 64-224 chunks).
 template <int FMT>
 __global__ __launch_bounds__(NT) void rw_col_finalize_kernel(const float *partial, int64_t nchunk,
                                                               int64_t inner, const float *scale_in,
                                                               float *scale, float *scale_inv) {
-    const int64_t n = static_cast<int64_t>(blockIdx.x) * NT + threadIdx.x;
-    const int64_t o = blockIdx.y;
-    if (n >= inner) return;
-    float sc;
-    if (scale_in != nullptr) {
-        sc = scale_in[o * inner + n];
-    } else {
-        float a = 0.0f;
-        for (int64_t c = 0; c < nchunk; ++c) a = fmaxf(a, partial[(o * nchunk + c) * inner + n]);
-        sc = scale_from_amax<FMT>(a, 1e-12f);
+    __shared__ float s[4][64];
+    const int     lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int64_t n = static_cast<int64_t>(blockIdx.x) * 64 + lane, o = blockIdx.y;
+    float         a = 0.0f;
+    if (scale_in == nullptr && n < inner) {
+#pragma unroll 4
+        for (int64_t c = part; c < nchunk; c += 4) a = amax2(a, partial[(o * nchunk + c) * inner + n]);
     }
+    s[part][lane] = a;
+    __syncthreads();
+    if (part != 0 || n >= inner) return;
+    a = amax2(amax2(s[0][lane], s[1][lane]), amax2(s[2][lane], s[3][lane]));
+    const float sc = scale_in != nullptr ? scale_in[o * inner + n] : scale_from_amax<FMT>(a, 1e-12f);
     scale[o * inner + n]     = sc;
     scale_inv[o * inner + n] = 1.0f / sc;
+}
+
+// Source of the vector column kernels: 8 consecutive columns of a row as fp32.
+// REQ false: x holds IN_DT elements.  REQ true: x holds fp8 bytes (SFMT) with one
+// scale per row, and an element enters as it would after a dequantization to
+// IN_DT: the fp32 product rounded to IN_DT.
+template <int IN_DT, bool REQ, int SFMT>
+__device__ __forceinline__ void rw_load8(const void *x, int64_t idx, float srow, float (&v)[8]) {
+    if constexpr (!REQ) {
+        load8<IN_DT>(x, idx, v);
+    } else {
+        const uint2 w = *reinterpret_cast<const uint2 *>(static_cast<const uint8_t *>(x) + idx);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int u = static_cast<int>(h == 0 ? w.x : w.y);
+            if constexpr (SFMT == PTA_E4M3) {
+                v[4 * h] = __builtin_amdgcn_cvt_f32_fp8(u, 0); v[4 * h + 1] = __builtin_amdgcn_cvt_f32_fp8(u, 1);
+                v[4 * h + 2] = __builtin_amdgcn_cvt_f32_fp8(u, 2); v[4 * h + 3] = __builtin_amdgcn_cvt_f32_fp8(u, 3);
+            } else {
+                v[4 * h] = __builtin_amdgcn_cvt_f32_bf8(u, 0); v[4 * h + 1] = __builtin_amdgcn_cvt_f32_bf8(u, 1);
+                v[4 * h + 2] = __builtin_amdgcn_cvt_f32_bf8(u, 2); v[4 * h + 3] = __builtin_amdgcn_cvt_f32_bf8(u, 3);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[j] *= srow;
+            if constexpr (IN_DT == PTA_BF16) v[j] = bf16_bits_to_f32(f32_to_bf16_bits(v[j]));
+            if constexpr (IN_DT == PTA_F16) v[j] = f16_bits_to_f32(f32_to_f16_bits(v[j]));
+        }
+    }
+}
+
+// Partial column amax, vector form: 512 columns x RW_CH rows per workgroup, 16
+// bytes (8 columns) per lane, the rows split over the 4 waves.
+template <int IN_DT, bool REQ, int SFMT>
+__global__ __launch_bounds__(NT) void rw_colv_partial_kernel(const void *x, const float *srow, int64_t len,
+                                                              int64_t inner, float *partial, int64_t nchunk) {
+    __shared__ __attribute__((aligned(16))) float s[4][512];
+    const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 512, n = n0 + lane * 8;
+    const int64_t c = blockIdx.y, o = blockIdx.z;
+    const int64_t r0 = c * RW_CH, r1 = r0 + RW_CH < len ? r0 + RW_CH : len;
+    float         m[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (n < inner) {
+#pragma unroll 8
+        for (int64_t r = r0 + wave; r < r1; r += 4) {
+            float v[8];
+            rw_load8<IN_DT, REQ, SFMT>(x, (o * len + r) * inner + n, REQ ? srow[r] : 0.0f, v);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], absq(v[j]));
+        }
+    }
+    *reinterpret_cast<float4 *>(&s[wave][lane * 8])     = make_float4(m[0], m[1], m[2], m[3]);
+    *reinterpret_cast<float4 *>(&s[wave][lane * 8 + 4]) = make_float4(m[4], m[5], m[6], m[7]);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = threadIdx.x + NT * h;
+        if (n0 + k < inner)
+            partial[(o * nchunk + c) * inner + n0 + k] = amax2(amax2(s[0][k], s[1][k]), amax2(s[2][k], s[3][k]));
+    }
+}
+
+// Quantize along the rows' axis, vector form: a 128 x 128 tile per workgroup, 4
+// rows x 16 columns per lane.  TRANS writes q[inner, len] (K-contiguous for a
+// GEMM that contracts over the rows): four rows of a column make one dword, the
+// tile passes through LDS as in byte_transpose.h.  Bound by memory; MI355X,
+// 8192 x 14336 bf16: amax + finalize + transposed quantize 43.5 + 5.4 + 67 us
+// (124 + 33 + 149 us with one element per lane and load, plus 42 us for the byte
+// transpose).  Re-quantizing 14336 x 4096 fp8 rows: 26 + 5.5 + 30 us, where the
+// dequantized copy cost 28 + 42 + 55 + 49 us and the byte transpose 23 us.
+template <int IN_DT, bool REQ, int SFMT, int FMT, bool TRANS>
+__global__ __launch_bounds__(NT) void rw_colv_quant_kernel(const void *x, const float *srow, int64_t len,
+                                                            int64_t inner, const float *scale, uint8_t *q) {
+    __shared__ __attribute__((aligned(16))) uint32_t s[TRANS ? 128 : 1][32];
+    const int     t = threadIdx.x, cseg = t & 7, rg = t >> 3;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 128, m0 = static_cast<int64_t>(blockIdx.y) * 128, o = blockIdx.z;
+    const int     rows = static_cast<int>(len - m0 < 128 ? len - m0 : 128);
+    const int     cols = static_cast<int>(inner - n0 < 128 ? inner - n0 : 128); // a multiple of 16
+    const bool    in   = cseg * 16 < cols;
+    const int64_t n    = n0 + cseg * 16;
+    float         v[4][16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * rg + i;
+        float     a[8], b[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = b[j] = 0.0f;
+        if (in && r < rows) {
+            const int64_t idx = (o * len + m0 + r) * inner + n;
+            const float   sr  = REQ ? srow[m0 + r] : 0.0f;
+            rw_load8<IN_DT, REQ, SFMT>(x, idx, sr, a);
+            rw_load8<IN_DT, REQ, SFMT>(x, idx + 8, sr, b);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { v[i][j] = a[j]; v[i][8 + j] = b[j]; }
+    }
+    float sc[16];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float4 f = in ? *reinterpret_cast<const float4 *>(scale + o * inner + n + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
+        sc[4 * j] = f.x; sc[4 * j + 1] = f.y; sc[4 * j + 2] = f.z; sc[4 * j + 3] = f.w;
+    }
+    if constexpr (!TRANS) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * rg + i;
+            if (!in || r >= rows) continue;
+            uint32_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                w[j] = qpack4s<FMT>(v[i][4 * j], v[i][4 * j + 1], v[i][4 * j + 2], v[i][4 * j + 3], sc[4 * j],
+                                    sc[4 * j + 1], sc[4 * j + 2], sc[4 * j + 3]);
+            *reinterpret_cast<uint4 *>(q + (o * len + m0 + r) * inner + n) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            s[cseg * 16 + j][rg ^ (cseg << 2)] = qpack4<FMT>(v[0][j], v[1][j], v[2][j], v[3][j], sc[j]);
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            const int c = it * 32 + (t >> 3), k = t & 7; // output row, its 16-byte chunk (len % 16 == 0)
+            if (c < cols && k * 16 < rows)
+                *reinterpret_cast<uint4 *>(q + (o * inner + n0 + c) * len + m0 + k * 16) =
+                    *reinterpret_cast<const uint4 *>(&s[c][(k ^ ((c >> 4) & 7)) << 2]);
+        }
+    }
 }
 
 template <int IN_DT, int FMT>
@@ -1127,9 +1259,34 @@ int rw_last_launch(const void *x, int64_t rows, int64_t len, const float *scale,
     return PTA_OK;
 }
 
+// columns quantized by the vector kernels: whole 16-column segments, aligned
+template <int IN_DT, bool REQ, int SFMT, int FMT, bool TRANS>
+int rw_colv_launch(const void *x, const float *srow, int64_t outer, int64_t len, int64_t inner, const float *scale_in,
+                   uint8_t *q, float *scale_inv, float *ws, hipStream_t st) {
+    const int64_t nchunk  = cdiv(len, RW_CH);
+    float        *scale   = ws;
+    float        *partial = ws + outer * inner;
+    const uint32_t no     = static_cast<uint32_t>(outer);
+    if (scale_in == nullptr) {
+        const dim3 g(static_cast<uint32_t>(cdiv(inner, 512)), static_cast<uint32_t>(nchunk), no);
+        rw_colv_partial_kernel<IN_DT, REQ, SFMT><<<g, NT, 0, st>>>(x, srow, len, inner, partial, nchunk);
+        PTA_CHECK_LAUNCH();
+    }
+    rw_col_finalize_kernel<FMT><<<dim3(static_cast<uint32_t>(cdiv(inner, 64)), no), NT, 0, st>>>(
+        partial, nchunk, inner, scale_in, scale, scale_inv);
+    PTA_CHECK_LAUNCH();
+    const dim3 g(static_cast<uint32_t>(cdiv(inner, 128)), static_cast<uint32_t>(cdiv(len, 128)), no);
+    rw_colv_quant_kernel<IN_DT, REQ, SFMT, FMT, TRANS><<<g, NT, 0, st>>>(x, srow, len, inner, scale, q);
+    PTA_CHECK_LAUNCH();
+    return PTA_OK;
+}
+
 template <int IN_DT, int FMT>
 int rw_col_launch(const void *x, int64_t outer, int64_t len, int64_t inner, const float *scale_in,
                   uint8_t *q, float *scale_inv, float *ws, hipStream_t st) {
+    // ws + outer * inner floats: 16-byte aligned scales need inner % 4 == 0 and an aligned workspace
+    if (inner % 16 == 0 && aligned16(x) && aligned16(q) && aligned16(ws))
+        return rw_colv_launch<IN_DT, false, 0, FMT, false>(x, nullptr, outer, len, inner, scale_in, q, scale_inv, ws, st);
     const int64_t nchunk  = cdiv(len, RW_CH);
     float        *scale   = ws;
     float        *partial = ws + outer * inner;
@@ -1139,12 +1296,22 @@ int rw_col_launch(const void *x, int64_t outer, int64_t len, int64_t inner, cons
         rw_col_partial_kernel<IN_DT><<<g3, NT, 0, st>>>(x, len, inner, partial, nchunk);
         PTA_CHECK_LAUNCH();
     }
-    rw_col_finalize_kernel<FMT><<<dim3(static_cast<uint32_t>(cdiv(inner, NT)), static_cast<uint32_t>(outer)), NT, 0, st>>>(
+    rw_col_finalize_kernel<FMT><<<dim3(static_cast<uint32_t>(cdiv(inner, 64)), static_cast<uint32_t>(outer)), NT, 0, st>>>(
         partial, nchunk, inner, scale_in, scale, scale_inv);
     PTA_CHECK_LAUNCH();
     rw_col_quant_kernel<IN_DT, FMT><<<g3, NT, 0, st>>>(x, len, inner, scale, q);
     PTA_CHECK_LAUNCH();
     return PTA_OK;
+}
+
+template <int IN_DT, int FMT>
+int rw_col_t_launch(const void *x, int src_fmt, const float *src_scale, int64_t M, int64_t N, uint8_t *q_t,
+                    float *scale_inv, float *ws, hipStream_t st) {
+    if (src_scale == nullptr)
+        return rw_colv_launch<IN_DT, false, 0, FMT, true>(x, nullptr, 1, M, N, nullptr, q_t, scale_inv, ws, st);
+    if (src_fmt == PTA_E4M3)
+        return rw_colv_launch<IN_DT, true, PTA_E4M3, FMT, true>(x, src_scale, 1, M, N, nullptr, q_t, scale_inv, ws, st);
+    return rw_colv_launch<IN_DT, true, PTA_E5M2, FMT, true>(x, src_scale, 1, M, N, nullptr, q_t, scale_inv, ws, st);
 }
 
 int check_in(const void *x, int in_dtype, int fmt) {
@@ -1278,6 +1445,23 @@ extern "C" int pta_quantize_fp8_rowwise(const void *x, int in_dtype, int64_t out
     return PTA_DISPATCH_IN_FMT(in_dtype, fmt, rw_col_launch, x, outer, len, inner, scale,
                                static_cast<uint8_t *>(q), scale_inv,
                                static_cast<float *>(workspace), st);
+}
+
+extern "C" int pta_quantize_fp8_rowwise_cols_t(const void *x, int in_dtype, int src_fmt, const float *src_scale,
+                                               int64_t M, int64_t N, void *q_t, int fmt, float *scale_inv,
+                                               void *workspace, size_t workspace_bytes, pta_stream_t stream) {
+    clear_error();
+    if (int rc = check_in(x, in_dtype, fmt)) return rc;
+    PTA_CHECK_ARG(q_t && scale_inv && M >= 0 && N >= 0, "bad arguments");
+    PTA_CHECK_ARG(src_scale == nullptr || src_fmt == PTA_E4M3 || src_fmt == PTA_E5M2, "unsupported source fp8 format");
+    PTA_CHECK_ARG(M % 16 == 0 && N % 16 == 0, "M and N must be multiples of 16");
+    PTA_CHECK_ARG(cdiv(M, RW_CH) <= 65535, "shape too large");
+    PTA_CHECK_ARG(aligned16(x) && aligned16(q_t) && aligned16(workspace), "buffers must be 16-byte aligned");
+    if (M == 0 || N == 0) return PTA_OK;
+    const size_t need = pta_quantize_fp8_rowwise_workspace_size(1, M, N);
+    PTA_CHECK_ARG(workspace_bytes >= need && workspace, "workspace of %zu bytes required", need);
+    return PTA_DISPATCH_IN_FMT(in_dtype, fmt, rw_col_t_launch, x, src_fmt, src_scale, M, N,
+                               static_cast<uint8_t *>(q_t), scale_inv, static_cast<float *>(workspace), as_stream(stream));
 }
 
 extern "C" int pta_quantize_mxfp8(const void *x, int in_dtype, int64_t G, int64_t M, int64_t N,

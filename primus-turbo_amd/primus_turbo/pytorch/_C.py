@@ -39,6 +39,7 @@ SIGNATURES = {
     "pta_quantize_fp8_tensorwise_noalloc": (_i32, [_vp, _i32, _i64, _vp, _vp, _i32, _vp, _vp]),
     "pta_quantize_fp8_rowwise_workspace_size": (_sz, [_i64, _i64, _i64]),
     "pta_quantize_fp8_rowwise": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _i32, _vp, _vp, _sz, _vp]),
+    "pta_quantize_fp8_rowwise_cols_t": (_i32, [_vp, _i32, _i32, _vp, _i64, _i64, _vp, _i32, _vp, _vp, _sz, _vp]),
     "pta_quantize_fp8_blockwise": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _i32, _vp]),
     "pta_quantize_fp8_blockwise_dual": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "pta_quantize_fp8_blockwise_for_weight": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp]),

@@ -87,6 +87,28 @@ def quantize_fp8_rowwise_impl(
     return q, scale_inv
 
 
+def quantize_fp8_rowwise_cols_t_impl(
+    x: torch.Tensor, out_dtype: torch.dtype, src_scale: Optional[torch.Tensor] = None,
+    src_dtype: Optional[torch.dtype] = None,
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """ROWWISE quantization of ``x`` [M, N] along axis 0 with the bytes written
+    transposed: (q_t [N, M], scale_inv [N]).  M and N are multiples of 16.  With
+    ``src_scale`` (one value per row) ``x`` is an fp8 tensor, re-quantized as its
+    dequantization to ``src_dtype`` would be."""
+    M, N = x.shape
+    x = x.contiguous()
+    q_t = torch.empty((N, M), dtype=out_dtype, device=x.device)
+    scale_inv = torch.empty((N,), dtype=torch.float32, device=x.device)
+    ws = _C.workspace(_C.query("pta_quantize_fp8_rowwise_workspace_size", 1, M, N), x.device)
+    in_code = _C.in_dtype_code(x.dtype if src_scale is None else src_dtype)
+    src_fmt = 0 if src_scale is None else _C.fp8_code(x.dtype)
+    _C.call(
+        "pta_quantize_fp8_rowwise_cols_t", _C.ptr(x), in_code, src_fmt, _C.ptr(src_scale), M, N, _C.ptr(q_t),
+        _C.fp8_code(out_dtype), _C.ptr(scale_inv), _C.ptr(ws), 0 if ws is None else ws.numel(), _C.stream(x.device),
+    )
+    return q_t, scale_inv
+
+
 def dequantize_fp8_tensorwise_impl(x: torch.Tensor, out_dtype: torch.dtype, scale_inv: torch.Tensor):
     x = x.contiguous()
     y = torch.empty(x.shape, dtype=out_dtype, device=x.device)

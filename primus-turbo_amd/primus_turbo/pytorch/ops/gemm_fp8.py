@@ -33,6 +33,7 @@ from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_impl, gemm_
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_impl,
     quant_fp8_blockwise_for_weight_impl,
+    quantize_fp8_rowwise_cols_t_impl,
     quantize_mxfp8_impl,
     transpose_fp8,
 )
@@ -151,6 +152,9 @@ class FP8GemmTensorFunction(torch.autograd.Function):
 # ===========================================================================
 # ROWWISE (gemm_fp8.py:231-379): the backward copies are re-quantized along
 # the other axis from the dequantized forward tensors, as in the reference.
+# Where M, N and K are multiples of 16, one call re-quantizes the fp8 bytes (the
+# dequantized copy stays in registers) and writes them K-contiguous for the
+# backward products, which then need no byte transposes.
 # ===========================================================================
 class FP8GemmRowFunction(torch.autograd.Function):
     @staticmethod
@@ -164,10 +168,18 @@ class FP8GemmRowFunction(torch.autograd.Function):
         else:
             qa = QuantizedTensor.quantize(a, _get_fp8_dtype(config.format, True), g, axis=-1,
                                           block_size=config.block_size)
-        if a_t is None:
+        M, K = a.shape
+        N = b.shape[0] if trans_b else b.shape[1]
+        whole = M % 16 == 0 and N % 16 == 0 and K % 16 == 0
+        a_cols = a_t is None and whole  # a's backward copy as [K, M] columns
+        b_cols = b_t is None and whole and trans_b  # b's as [K, N]
+        if a_cols:
+            a_bwd = quantize_fp8_rowwise_cols_t_impl(qa.qdata, qa.real_dtype, qa.scale_inv, qa.dtype)
+        elif a_t is None:
             qa_t = QuantizedTensor.quantize(qa.dequantize(), qa.real_dtype, g, axis=-2, block_size=config.block_size)
+            a_bwd = qa_t.qdata, qa_t.scale_inv
         else:
-            qa_t = a_t
+            a_bwd = a_t.qdata, a_t.scale_inv
         b_axis = -1 if trans_b else -2
         if isinstance(b, QuantizedTensor):
             check_quantized_tensor(b, config, axis=b_axis)
@@ -175,13 +187,17 @@ class FP8GemmRowFunction(torch.autograd.Function):
         else:
             qb = QuantizedTensor.quantize(b, _get_fp8_dtype(config.format, True), g, axis=b_axis,
                                           block_size=config.block_size)
-        if b_t is None:
+        if b_cols:
+            b_bwd = quantize_fp8_rowwise_cols_t_impl(qb.qdata, qb.real_dtype, qb.scale_inv, qb.dtype)
+        elif b_t is None:
             qb_t = QuantizedTensor.quantize(qb.dequantize(), qb.real_dtype, g, axis=-2 if trans_b else -1,
                                             block_size=config.block_size)
+            b_bwd = qb_t.qdata, qb_t.scale_inv
         else:
-            qb_t = b_t
+            b_bwd = b_t.qdata, b_t.scale_inv
         out = _nt_or_impl(qa.qdata, qa.scale_inv, trans_a, qb.qdata, qb.scale_inv, trans_b, out_dtype, False, g)
-        ctx.save_for_backward(qa_t.qdata, qa_t.scale_inv, qb_t.qdata, qb_t.scale_inv)
+        ctx.save_for_backward(*a_bwd, *b_bwd)
+        ctx.a_cols, ctx.b_cols = a_cols, b_cols
         ctx.trans_a, ctx.trans_b, ctx.out_dtype, ctx.config = trans_a, trans_b, out_dtype, config
         return out
 
@@ -193,10 +209,17 @@ class FP8GemmRowFunction(torch.autograd.Function):
         a_t, a_t_s, b_t, b_t_s = ctx.saved_tensors
         gd = _get_fp8_dtype(ctx.config.format, False)
         qg = QuantizedTensor.quantize(grad_out, gd, g, axis=-1, block_size=ctx.config.block_size)
-        a_grad = _nt_or_impl(qg.qdata, qg.scale_inv, False, b_t, b_t_s, not ctx.trans_b, ctx.out_dtype, ctx.trans_a, g)
-        qg_t = QuantizedTensor.quantize(grad_out, gd, g, axis=-2, block_size=ctx.config.block_size)
-        b_grad = _nt_or_impl(a_t, a_t_s, not ctx.trans_a, qg_t.qdata, qg_t.scale_inv, False, ctx.out_dtype,
-                             ctx.trans_b, g)
+        # dgrad over N: b's copy is [K, N] columns, or stored as b with the other axis' scales
+        a_grad = _nt_or_impl(qg.qdata, qg.scale_inv, False, b_t, b_t_s, ctx.b_cols or not ctx.trans_b, ctx.out_dtype,
+                             ctx.trans_a, g)
+        if ctx.a_cols:  # wgrad over M: dW[N, K] = g_cols . a_cols^T, or its transpose
+            g_cols, g_s = quantize_fp8_rowwise_cols_t_impl(grad_out, gd)
+            lhs, rhs = ((g_cols, g_s), (a_t, a_t_s)) if ctx.trans_b else ((a_t, a_t_s), (g_cols, g_s))
+            b_grad = _nt_or_impl(*lhs, False, *rhs, True, ctx.out_dtype, False, g)
+        else:
+            qg_t = QuantizedTensor.quantize(grad_out, gd, g, axis=-2, block_size=ctx.config.block_size)
+            b_grad = _nt_or_impl(a_t, a_t_s, not ctx.trans_a, qg_t.qdata, qg_t.scale_inv, False, ctx.out_dtype,
+                                 ctx.trans_b, g)
         return a_grad, b_grad, None, None, None, None, None, None
 
 

@@ -78,3 +78,37 @@ def test_dequant_routes_agree_with_the_definition(shape, out_dtype):
     y = dequantize_fp8(q, out_dtype, ScalingGranularity.BLOCKWISE, block_size=128, scale_inv=s, scaling_recipe=recipe)
     wide = s.repeat_interleave(128, 1).repeat_interleave(128, 2)[:, : shape[0], : shape[1]]
     assert torch.equal(y.cpu(), want(q, wide))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fmt", [E4, torch.float8_e5m2])
+@pytest.mark.parametrize("shape", [(16, 16), (128, 128), (144, 272), (1040, 528), (4096, 512)])
+def test_rowwise_columns_transposed(shape, fmt, dtype):
+    """The column quantization that writes transposed bytes, from high-precision
+    rows and from fp8 rows, against the definition (quotients rounded once)."""
+    from primus_turbo.pytorch.kernels.quantization.quantization_impl import quantize_fp8_rowwise_cols_t_impl
+
+    g = torch.Generator().manual_seed(shape[0])
+    x = (torch.randn(shape, generator=g) * torch.logspace(-6, 3, shape[1])).to(dtype)
+    x[:, 1] = 0
+    x[0, 2], x[1, 2], x[0, 3] = float("inf"), -float("inf"), float("nan")
+    top = torch.finfo(fmt).max
+
+    def want(v):
+        a = v.float().abs().nan_to_num(nan=0.0, posinf=float("inf")).amax(0)
+        s = (top / a.clamp(min=1e-12).double()).float()
+        p = v.float() * s
+        q = torch.where(p.isnan(), torch.full_like(p, top), p).clamp(-top, top).to(fmt)
+        return q.t().contiguous().view(torch.uint8), (1.0 / s.double()).float()
+
+    q, s = quantize_fp8_rowwise_cols_t_impl(x.cuda(), fmt)
+    wq, ws = want(x)
+    assert torch.equal(q.view(torch.uint8).cpu(), wq) and torch.equal(s.cpu(), ws)
+    plain = quantize_fp8(x.cuda(), fmt, ScalingGranularity.ROWWISE, axis=0)
+    assert torch.equal(plain[0].view(torch.uint8).cpu(), wq.t()) and torch.equal(plain[1].cpu().view(-1), ws)
+    # fp8 rows with a scale each: as their dequantization to dtype
+    x = torch.nan_to_num(x.float(), nan=1.0, posinf=2.0, neginf=-2.0).to(dtype)
+    r, rs = quantize_fp8(x.cuda(), fmt, ScalingGranularity.ROWWISE, axis=1)
+    q, s = quantize_fp8_rowwise_cols_t_impl(r, fmt, rs, dtype)
+    wq, ws = want((r.float().cpu() * rs.cpu()).to(dtype))
+    assert torch.equal(q.view(torch.uint8).cpu(), wq) and torch.equal(s.cpu(), ws)
