@@ -129,13 +129,21 @@ class _Permute(torch.autograd.Function):
         sf = scaling_factor if use_fp8 else None
         rows, out_probs, out_sf = _expert_major(r, tokens, n_rows, probs, sf, scales_per_token, use_fp8)
         _save(ctx, r)
+        ctx.set_materialize_grads(False)  # no zero tensors for the index outputs
         ctx.n_tokens, ctx.fp8, ctx.has_probs = T, use_fp8, probs is not None
+        ctx.row_like = (n_rows, int(tokens.shape[-1]), tokens.dtype, tokens.device)
         return rows, r.row_id_map, tpe, ovf, r.num_dispatched, out_sf, out_probs
 
     @staticmethod
     def backward(ctx, g_rows, _g_map, _g_tpe, _g_ovf, _g_nd, _g_sf, g_probs):
         assert not ctx.fp8, "moe_permute: fp8 tokens have no backward"
-        g_probs = g_probs if ctx.has_probs else None
+        n_rows, H, dtype, dev = ctx.row_like
+        if g_rows is None:
+            g_rows = torch.zeros((n_rows, H), dtype=dtype, device=dev)
+        if not (ctx.has_probs and ctx.needs_input_grad[7]):
+            g_probs = None
+        elif g_probs is None:
+            g_probs = torch.zeros((n_rows,), dtype=torch.float32, device=dev)
         g_tokens, g_in_probs = _token_major(_load(ctx), g_rows, ctx.n_tokens, g_probs)
         return g_tokens, None, None, None, None, None, None, g_in_probs, None, None, None
 
