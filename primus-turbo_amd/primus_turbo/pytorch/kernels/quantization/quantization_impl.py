@@ -167,6 +167,7 @@ def quant_fp8_blockwise_dual_impl(
     block_size: int = 128,
     col_transposed: bool = False,
     row_scale_kmajor: bool = False,
+    row_only: bool = False,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """Row (1 x bs) and column (bs x 1) quantization in one read of ``x``.
 
@@ -178,6 +179,7 @@ def quant_fp8_blockwise_dual_impl(
     - ``row_scale_kmajor=True`` returns the row scales as a ``[M, N/bs]`` view
       of ``[N/bs, M]`` storage (strides ``(1, M)``): the GEMM then reads the
       scales of one K block for 16 consecutive rows from one cache line.
+    ``row_only=True`` leaves the column outputs out (None).
     """
     _check_hp(x)
     assert x.is_contiguous() and x.dim() == 2, "Input must be 2D and contiguous"
@@ -188,8 +190,10 @@ def quant_fp8_blockwise_dual_impl(
         s_row = torch.empty((nb, M), dtype=torch.float32, device=x.device).t()
     else:
         s_row = torch.empty((M, nb), dtype=torch.float32, device=x.device)
-    q_col = torch.empty((N, ceil_div(M, 128) * 128) if col_transposed else (M, N), dtype=dtype, device=x.device)
-    s_col = torch.empty((ceil_div(M, block_size), N), dtype=torch.float32, device=x.device)
+    q_col = s_col = None
+    if not row_only:
+        q_col = torch.empty((N, ceil_div(M, 128) * 128) if col_transposed else (M, N), dtype=dtype, device=x.device)
+        s_col = torch.empty((ceil_div(M, block_size), N), dtype=torch.float32, device=x.device)
     layout = (_C.DUAL_COL_TRANSPOSED if col_transposed else 0) | (_C.DUAL_ROW_SCALE_KMAJOR if row_scale_kmajor else 0)
     _C.call(
         "pta_quantize_fp8_blockwise_dual", _C.ptr(x), _C.in_dtype_code(x.dtype), M, N, block_size, _C.ptr(q_row),

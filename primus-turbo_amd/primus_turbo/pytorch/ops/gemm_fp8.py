@@ -31,9 +31,12 @@ from primus_turbo.pytorch.core.quantized_tensor import (
 )
 from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_impl, gemm_fp8_nt
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
+    dequantize_fp8_rowwise_impl,
     quant_fp8_blockwise_dual_impl,
     quant_fp8_blockwise_for_weight_impl,
     quantize_fp8_rowwise_cols_t_impl,
+    quantize_fp8_rowwise_impl,
+    quantize_fp8_tensorwise_impl,
     quantize_mxfp8_impl,
     transpose_fp8,
 )
@@ -104,29 +107,40 @@ def _nt_or_impl(a, sa, trans_a, b, sb, trans_b, out_dtype, trans_c, gran: Scalin
 # ===========================================================================
 # TENSORWISE
 # ===========================================================================
+def _tensorwise(x, dtype, config):
+    """(fp8 data, scale) of an operand: an already quantized one as it is."""
+    if isinstance(x, QuantizedTensor):
+        check_quantized_tensor(x, config)
+        return x.qdata, x.scale_inv
+    return quantize_fp8_tensorwise_impl(x, dtype)
+
+
+def _tensorwise_t(x, x_t, q, s):
+    """The transposed copy that the NT backward reads: the caller's, or q's."""
+    if isinstance(x_t, QuantizedTensor):
+        return x_t.qdata, x_t.scale_inv
+    if isinstance(x, QuantizedTensor):
+        x_t = x.t()
+        return x_t.qdata, x_t.scale_inv
+    return transpose_fp8(q), s
+
+
 class FP8GemmTensorFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config):
+    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, need_bwd):
         _refuse_capture()
         g = ScalingGranularity.TENSORWISE
         nt_bwd = _use_nt_layout_gemm_in_bwd(trans_a, trans_b)
-        if isinstance(a, QuantizedTensor):
-            qa = a
-            check_quantized_tensor(qa, config)
-        else:
-            qa = QuantizedTensor.quantize(a, _get_fp8_dtype(config.format, True), g, axis=-1)
-        if isinstance(b, QuantizedTensor):
-            qb = b
-            check_quantized_tensor(qb, config)
-        else:
-            qb = QuantizedTensor.quantize(b, _get_fp8_dtype(config.format, True), g, axis=-1)
-        out = _nt_or_impl(qa.qdata, qa.scale_inv, trans_a, qb.qdata, qb.scale_inv, trans_b, out_dtype, False, g)
+        fdt = _get_fp8_dtype(config.format, True)
+        qa, sa = _tensorwise(a, fdt, config)
+        qb, sb = _tensorwise(b, fdt, config)
+        out = _nt_or_impl(qa, sa, trans_a, qb, sb, trans_b, out_dtype, False, g)
+        if not need_bwd:
+            return out
         if nt_bwd:
-            qa_t = a_t if isinstance(a_t, QuantizedTensor) else qa.t()
-            qb_t = b_t if isinstance(b_t, QuantizedTensor) else qb.t()
-            ctx.save_for_backward(qa_t.qdata, qa_t.scale_inv, qb_t.qdata, qb_t.scale_inv)
+            ctx.save_for_backward(*_tensorwise_t(a, a_t, qa, sa), *_tensorwise_t(b, b_t, qb, sb))
         else:
-            ctx.save_for_backward(qa.qdata, qa.scale_inv, qb.qdata, qb.scale_inv)
+            ctx.save_for_backward(qa, sa, qb, sb)
         ctx.trans_a, ctx.trans_b, ctx.out_dtype, ctx.config, ctx.nt_bwd = trans_a, trans_b, out_dtype, config, nt_bwd
         return out
 
@@ -136,17 +150,17 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         g = ScalingGranularity.TENSORWISE
         grad_out = grad_out.contiguous()
         x0, s0, x1, s1 = ctx.saved_tensors
-        qg = QuantizedTensor.quantize(grad_out, _get_fp8_dtype(ctx.config.format, False), g, axis=-1)
+        qg, sg = quantize_fp8_tensorwise_impl(grad_out, _get_fp8_dtype(ctx.config.format, False))
         if ctx.nt_bwd:
             a_t, a_t_s, b_t, b_t_s = x0, s0, x1, s1
-            a_grad = _nt_or_impl(qg.qdata, qg.scale_inv, False, b_t, b_t_s, True, ctx.out_dtype, False, g)
-            g_t = transpose_fp8(qg.qdata)
-            b_grad = _nt_or_impl(a_t, a_t_s, False, g_t, qg.scale_inv, True, ctx.out_dtype, ctx.trans_b, g)
+            a_grad = _nt_or_impl(qg, sg, False, b_t, b_t_s, True, ctx.out_dtype, False, g)
+            g_t = transpose_fp8(qg)
+            b_grad = _nt_or_impl(a_t, a_t_s, False, g_t, sg, True, ctx.out_dtype, ctx.trans_b, g)
         else:
             a8, sa, b8, sb = x0, s0, x1, s1
-            a_grad = _nt_or_impl(qg.qdata, qg.scale_inv, False, b8, sb, not ctx.trans_b, ctx.out_dtype, ctx.trans_a, g)
-            b_grad = _nt_or_impl(a8, sa, not ctx.trans_a, qg.qdata, qg.scale_inv, False, ctx.out_dtype, ctx.trans_b, g)
-        return a_grad, b_grad, None, None, None, None, None, None
+            a_grad = _nt_or_impl(qg, sg, False, b8, sb, not ctx.trans_b, ctx.out_dtype, ctx.trans_a, g)
+            b_grad = _nt_or_impl(a8, sa, not ctx.trans_a, qg, sg, False, ctx.out_dtype, ctx.trans_b, g)
+        return a_grad, b_grad, None, None, None, None, None, None, None
 
 
 # ===========================================================================
@@ -158,44 +172,44 @@ class FP8GemmTensorFunction(torch.autograd.Function):
 # ===========================================================================
 class FP8GemmRowFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config):
+    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, need_bwd):
         _refuse_capture()
         assert trans_a == False, "trans_a has to be False"
         g = ScalingGranularity.ROWWISE
+        fdt = _get_fp8_dtype(config.format, True)
         if isinstance(a, QuantizedTensor):
-            qa = a
-            check_quantized_tensor(qa, config, axis=-1)
+            check_quantized_tensor(a, config, axis=-1)
+            qa, sa, fa = a.qdata, a.scale_inv, a.real_dtype
         else:
-            qa = QuantizedTensor.quantize(a, _get_fp8_dtype(config.format, True), g, axis=-1,
-                                          block_size=config.block_size)
+            (qa, sa), fa = quantize_fp8_rowwise_impl(a, fdt, -1), fdt
+        b_axis = -1 if trans_b else -2
+        if isinstance(b, QuantizedTensor):
+            check_quantized_tensor(b, config, axis=b_axis)
+            qb, sb, fb = b.qdata, b.scale_inv, b.real_dtype
+        else:
+            (qb, sb), fb = quantize_fp8_rowwise_impl(b, fdt, b_axis), fdt
+        out = _nt_or_impl(qa, sa, trans_a, qb, sb, trans_b, out_dtype, False, g)
+        if not need_bwd:
+            return out
         M, K = a.shape
         N = b.shape[0] if trans_b else b.shape[1]
         whole = M % 16 == 0 and N % 16 == 0 and K % 16 == 0
         a_cols = a_t is None and whole  # a's backward copy as [K, M] columns
         b_cols = b_t is None and whole and trans_b  # b's as [K, N]
+
+        def again(q, s, dtype, fmt, row_axis):
+            """Dequantized and quantized along the other axis, in q's layout."""
+            x = dequantize_fp8_rowwise_impl(q, dtype, row_axis, s)
+            return quantize_fp8_rowwise_impl(x, fmt, -1 if row_axis % 2 == 0 else -2)
+
         if a_cols:
-            a_bwd = quantize_fp8_rowwise_cols_t_impl(qa.qdata, qa.real_dtype, qa.scale_inv, qa.dtype)
-        elif a_t is None:
-            qa_t = QuantizedTensor.quantize(qa.dequantize(), qa.real_dtype, g, axis=-2, block_size=config.block_size)
-            a_bwd = qa_t.qdata, qa_t.scale_inv
+            a_bwd = quantize_fp8_rowwise_cols_t_impl(qa, fa, sa, a.dtype)
         else:
-            a_bwd = a_t.qdata, a_t.scale_inv
-        b_axis = -1 if trans_b else -2
-        if isinstance(b, QuantizedTensor):
-            check_quantized_tensor(b, config, axis=b_axis)
-            qb = b
-        else:
-            qb = QuantizedTensor.quantize(b, _get_fp8_dtype(config.format, True), g, axis=b_axis,
-                                          block_size=config.block_size)
+            a_bwd = again(qa, sa, a.dtype, fa, 1) if a_t is None else (a_t.qdata, a_t.scale_inv)
         if b_cols:
-            b_bwd = quantize_fp8_rowwise_cols_t_impl(qb.qdata, qb.real_dtype, qb.scale_inv, qb.dtype)
-        elif b_t is None:
-            qb_t = QuantizedTensor.quantize(qb.dequantize(), qb.real_dtype, g, axis=-2 if trans_b else -1,
-                                            block_size=config.block_size)
-            b_bwd = qb_t.qdata, qb_t.scale_inv
+            b_bwd = quantize_fp8_rowwise_cols_t_impl(qb, fb, sb, b.dtype)
         else:
-            b_bwd = b_t.qdata, b_t.scale_inv
-        out = _nt_or_impl(qa.qdata, qa.scale_inv, trans_a, qb.qdata, qb.scale_inv, trans_b, out_dtype, False, g)
+            b_bwd = again(qb, sb, b.dtype, fb, b_axis) if b_t is None else (b_t.qdata, b_t.scale_inv)
         ctx.save_for_backward(*a_bwd, *b_bwd)
         ctx.a_cols, ctx.b_cols = a_cols, b_cols
         ctx.trans_a, ctx.trans_b, ctx.out_dtype, ctx.config = trans_a, trans_b, out_dtype, config
@@ -208,19 +222,17 @@ class FP8GemmRowFunction(torch.autograd.Function):
         grad_out = grad_out.contiguous()
         a_t, a_t_s, b_t, b_t_s = ctx.saved_tensors
         gd = _get_fp8_dtype(ctx.config.format, False)
-        qg = QuantizedTensor.quantize(grad_out, gd, g, axis=-1, block_size=ctx.config.block_size)
+        qg, sg = quantize_fp8_rowwise_impl(grad_out, gd, -1)
         # dgrad over N: b's copy is [K, N] columns, or stored as b with the other axis' scales
-        a_grad = _nt_or_impl(qg.qdata, qg.scale_inv, False, b_t, b_t_s, ctx.b_cols or not ctx.trans_b, ctx.out_dtype,
-                             ctx.trans_a, g)
+        a_grad = _nt_or_impl(qg, sg, False, b_t, b_t_s, ctx.b_cols or not ctx.trans_b, ctx.out_dtype, ctx.trans_a, g)
         if ctx.a_cols:  # wgrad over M: dW[N, K] = g_cols . a_cols^T, or its transpose
             g_cols, g_s = quantize_fp8_rowwise_cols_t_impl(grad_out, gd)
             lhs, rhs = ((g_cols, g_s), (a_t, a_t_s)) if ctx.trans_b else ((a_t, a_t_s), (g_cols, g_s))
             b_grad = _nt_or_impl(*lhs, False, *rhs, True, ctx.out_dtype, False, g)
         else:
-            qg_t = QuantizedTensor.quantize(grad_out, gd, g, axis=-2, block_size=ctx.config.block_size)
-            b_grad = _nt_or_impl(a_t, a_t_s, not ctx.trans_a, qg_t.qdata, qg_t.scale_inv, False, ctx.out_dtype,
-                                 ctx.trans_b, g)
-        return a_grad, b_grad, None, None, None, None, None, None
+            qg_t, sg_t = quantize_fp8_rowwise_impl(grad_out, gd, -2)
+            b_grad = _nt_or_impl(a_t, a_t_s, not ctx.trans_a, qg_t, sg_t, False, ctx.out_dtype, ctx.trans_b, g)
+        return a_grad, b_grad, None, None, None, None, None, None, None
 
 
 # ===========================================================================
@@ -234,7 +246,7 @@ def _weight_nk_kn(qw: torch.Tensor, trans_b: bool):
 
 class FP8GemmBlockFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config):
+    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, need_bwd):
         _refuse_capture()
         assert trans_a == False, "trans_a has to be False"
         assert config.block_size == _BLOCK, "BLOCKWISE supports block_size 128"
@@ -245,26 +257,29 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         if isinstance(a, QuantizedTensor):
             check_quantized_tensor(a, config, axis=-1)
             a_row, a_row_s = a.qdata, a.scale_inv
-            if a_t is None:
-                a_t = QuantizedTensor.quantize(a.dequantize(), fdt, gran, axis=-2, block_size=config.block_size)
-            a_colT = _pad_cols(transpose_fp8(a_t.qdata), _BLOCK)
-            a_col_s = a_t.scale_inv
+            if need_bwd:
+                if a_t is None:
+                    a_t = QuantizedTensor.quantize(a.dequantize(), fdt, gran, axis=-2, block_size=config.block_size)
+                a_colT = _pad_cols(transpose_fp8(a_t.qdata), _BLOCK)
+                a_col_s = a_t.scale_inv
         else:
             a_row, a_row_s, a_colT, a_col_s = quant_fp8_blockwise_dual_impl(
                 a.detach().contiguous(), fdt, block_size=config.block_size, col_transposed=True,
-                row_scale_kmajor=True,
+                row_scale_kmajor=True, row_only=not need_bwd,
             )
         # --- B: 128 x 128 blocks, reused by fwd and dgrad
         recipe = ScalingRecipe(use_2d_block=True)
         if isinstance(b, QuantizedTensor):
             check_quantized_tensor(b, config, scaling_recipe=recipe)
-            w_nk, w_kn = _weight_nk_kn(b.qdata, trans_b)
+            w_nk, w_kn = _weight_nk_kn(b.qdata, trans_b) if need_bwd or not trans_b else (b.qdata, None)
             w_s = b.scale_inv
-        else:
+        elif need_bwd or not trans_b:
             qw, w_s, qw_t = quant_fp8_blockwise_for_weight_impl(
                 b.detach().contiguous(), fdt, block_size=config.block_size, with_transpose=True
             )
             w_nk, w_kn = (qw, qw_t) if trans_b else (qw_t, qw)
+        else:
+            w_nk, w_s = quant_fp8_blockwise_for_weight_impl(b.detach().contiguous(), fdt, block_size=config.block_size)
         N = w_nk.shape[0]
         a_row = _pad_cols16(a_row)
         w_nk = _pad_cols16(w_nk)
@@ -274,6 +289,8 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         w_str_nk = (nbk, 1) if trans_b else (1, nbn)  # rows n, blocks k
         w_str_kn = (1, nbk) if trans_b else (nbn, 1)  # rows k, blocks n
         out = gemm_fp8_nt(a_row, w_nk, out_dtype, gran, a_row_s, a_row_s.stride(), False, w_s, w_str_nk, True)
+        if not need_bwd:
+            return out
         ctx.save_for_backward(a_colT, a_col_s, _pad_cols(w_kn, _BLOCK), w_s)
         ctx.w_str_kn = w_str_kn
         ctx.trans_b, ctx.out_dtype, ctx.config = trans_b, out_dtype, config
@@ -299,7 +316,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
             grad_b = gemm_fp8_nt(g_colT, a_colT, ctx.out_dtype, gran, g_col_s, (1, N), False, a_col_s, (1, K), False)
         else:  # dW[K, N]
             grad_b = gemm_fp8_nt(a_colT, g_colT, ctx.out_dtype, gran, a_col_s, (1, K), False, g_col_s, (1, N), False)
-        return grad_a, grad_b, None, None, None, None, None, None
+        return grad_a, grad_b, None, None, None, None, None, None, None
 
 
 # ===========================================================================
@@ -322,7 +339,7 @@ def _mx_gemm(a_q, a_e, b_q, b_e, out_dtype):
 
 class FP8GemmMXFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config):
+    def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, need_bwd):
         _refuse_capture()
         ok, reason = check_mxfp8_support()
         assert ok, reason
@@ -333,10 +350,13 @@ class FP8GemmMXFunction(torch.autograd.Function):
         if isinstance(a, QuantizedTensor):
             check_quantized_tensor(a, config, axis=-1, scaling_recipe=ra)
             a_row, a_row_s = a.qdata, a.scale_inv
-            if a_t is None:
-                a_t = QuantizedTensor.quantize(a.dequantize(), a.real_dtype, gran, axis=-2, block_size=bs,
-                                               scaling_recipe=ra)
-            a_col, a_col_s = a_t.qdata, a_t.scale_inv
+            if need_bwd:
+                if a_t is None:
+                    a_t = QuantizedTensor.quantize(a.dequantize(), a.real_dtype, gran, axis=-2, block_size=bs,
+                                                   scaling_recipe=ra)
+                a_col, a_col_s = a_t.qdata, a_t.scale_inv
+        elif not need_bwd:
+            a_row, a_row_s = quantize_mxfp8_impl(a.detach(), fdt, 1, bs, scaling_recipe=ra, exp_kmajor=True)
         else:
             a_row, a_row_s, a_col, a_col_s = quantize_mxfp8_impl(a.detach(), fdt, None, bs, with_trans=True,
                                                                  scaling_recipe=ra, scaling_recipe_for_trans=ra,
@@ -345,16 +365,21 @@ class FP8GemmMXFunction(torch.autograd.Function):
         if isinstance(b, QuantizedTensor):
             check_quantized_tensor(b, config, axis=-1, scaling_recipe=rb)
             b_row, b_row_s = b.qdata, b.scale_inv
-            if b_t is None:
-                b_t = QuantizedTensor.quantize(b.dequantize(), b.real_dtype, gran, axis=-2, block_size=bs,
-                                               scaling_recipe=rb)
-            b_col, b_col_s = b_t.qdata, b_t.scale_inv
+            if need_bwd:
+                if b_t is None:
+                    b_t = QuantizedTensor.quantize(b.dequantize(), b.real_dtype, gran, axis=-2, block_size=bs,
+                                                   scaling_recipe=rb)
+                b_col, b_col_s = b_t.qdata, b_t.scale_inv
+        elif not need_bwd:
+            b_row, b_row_s = quantize_mxfp8_impl(b.detach(), fdt, 1, bs, scaling_recipe=rb, exp_kmajor=True)
         else:
             b_row, b_row_s, b_col, b_col_s = quantize_mxfp8_impl(
                 b.detach(), fdt, None, bs, with_trans=True, scaling_recipe=rb, scaling_recipe_for_trans=rb,
                 exp_kmajor=True,
             )
         out = _mx_gemm(a_row, a_row_s, b_row, b_row_s, out_dtype)
+        if not need_bwd:
+            return out
         ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s)
         ctx.out_dtype, ctx.config = out_dtype, config
         ctx.M, ctx.N, ctx.K = a.shape[0], b.shape[0], a.shape[1]
@@ -371,7 +396,7 @@ class FP8GemmMXFunction(torch.autograd.Function):
         )
         grad_a = _mx_gemm(g_row, g_row_s, b_col, b_col_s, ctx.out_dtype)  # [M, K]
         grad_b = _mx_gemm(g_col, g_col_s, a_col, a_col_s, ctx.out_dtype)  # [N, K]
-        return grad_a[: ctx.M, : ctx.K], grad_b[: ctx.N, : ctx.K], None, None, None, None, None, None
+        return grad_a[: ctx.M, : ctx.K], grad_b[: ctx.N, : ctx.K], None, None, None, None, None, None, None
 
 
 @torch._dynamo.disable(recursive=True)
@@ -396,7 +421,10 @@ def gemm_fp8(
     assert b_data.ndim == 2, "Only 2D tensors are supported"
     if out_dtype is None:
         out_dtype = torch.promote_types(a_data.dtype, b_data.dtype)
-    args = (a_data, b_data, a_data_t, b_data_t, trans_a, trans_b, out_dtype, config)
+    # a call that no gradient can follow makes no backward copies
+    need_bwd = torch.is_grad_enabled() and any(
+        t is not None and t.requires_grad for t in (a_data, b_data, a_data_t, b_data_t))
+    args = (a_data, b_data, a_data_t, b_data_t, trans_a, trans_b, out_dtype, config, need_bwd)
     if config.granularity == ScalingGranularity.TENSORWISE:
         return FP8GemmTensorFunction.apply(*args)
     elif config.granularity == ScalingGranularity.ROWWISE:

@@ -33,8 +33,8 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     grouped_quantize_mxfp8_impl,
     quant_fp8_blockwise_for_weight_impl,
     quant_fp8_blockwise_segment_m_row_col_impl,
+    quantize_fp8_tensorwise_impl,
     quantize_mxfp8_impl,
-    transpose_fp8,
 )
 
 __all__ = ["grouped_gemm_fp8"]
@@ -163,26 +163,31 @@ class FP8GroupedGemmTensorFunc(torch.autograd.Function):
     """TENSORWISE (grouped_gemm_fp8.py:382-567)."""
 
     @staticmethod
-    def forward(ctx, a, b, a_t, b_t, group_lens, group_offs, trans_b, out_dtype, config, num_cu):
+    def forward(ctx, a, b, a_t, b_t, group_lens, group_offs, trans_b, out_dtype, config, num_cu, need_bwd):
         g = ScalingGranularity.TENSORWISE
         nt_bwd = trans_b
         if isinstance(a, QuantizedTensor):
             check_quantized_tensor(a, config)
-            qa = a
+            qa, sa = a.qdata, a.scale_inv
         else:
-            qa = QuantizedTensor.quantize(a, _get_fp8_dtype(config.format, True), g, axis=-1, group_lens=group_lens)
+            # (the group arrays belong to the call: none are made for the operand)
+            assert a.ndim == 2, f"Grouped quantized tensor expects a 2D packed-M tensor, got {a.ndim}D"
+            assert group_lens.is_cuda, "group_lens must be on CUDA"
+            qa, sa = quantize_fp8_tensorwise_impl(a, _get_fp8_dtype(config.format, True))
         if isinstance(b, QuantizedTensor):
             check_quantized_tensor(b, config)
             qb = b
         else:
             qb = QuantizedTensor.quantize(b, _get_fp8_dtype(config.format, True), g, axis=-1)
-        out = grouped_gemm_fp8_impl(qa.qdata, qb.qdata, qa.scale_inv, qb.scale_inv, group_lens, group_offs, False,
+        out = grouped_gemm_fp8_impl(qa, qb.qdata, sa, qb.scale_inv, group_lens, group_offs, False,
                                     trans_b, out_dtype, g.value, num_cu)
+        if not need_bwd:
+            return out
         if nt_bwd:
             qb_t = b_t if isinstance(b_t, QuantizedTensor) else qb.transpose(-1, -2)
-            ctx.save_for_backward(qa.qdata, qb_t.qdata, qa.scale_inv, qb_t.scale_inv, group_lens, group_offs)
+            ctx.save_for_backward(qa, qb_t.qdata, sa, qb_t.scale_inv, group_lens, group_offs)
         else:
-            ctx.save_for_backward(qa.qdata, qb.qdata, qa.scale_inv, qb.scale_inv, group_lens, group_offs)
+            ctx.save_for_backward(qa, qb.qdata, sa, qb.scale_inv, group_lens, group_offs)
         ctx.trans_b, ctx.nt_bwd, ctx.config, ctx.out_dtype, ctx.num_cu = trans_b, nt_bwd, config, out_dtype, num_cu
         return out
 
@@ -191,13 +196,13 @@ class FP8GroupedGemmTensorFunc(torch.autograd.Function):
         g = ScalingGranularity.TENSORWISE
         a8, b8, sa, sb, group_lens, group_offs = ctx.saved_tensors
         gdt = _get_fp8_dtype(ctx.config.format, False)
-        qg = QuantizedTensor.quantize(grad_out.contiguous(), gdt, g, axis=-1, group_lens=group_lens)
+        qg, sg = quantize_fp8_tensorwise_impl(grad_out.contiguous(), gdt)
         trans = True if ctx.nt_bwd else (not ctx.trans_b)
-        grad_a = grouped_gemm_fp8_impl(qg.qdata, b8, qg.scale_inv, sb, group_lens, group_offs, False, trans,
+        grad_a = grouped_gemm_fp8_impl(qg, b8, sg, sb, group_lens, group_offs, False, trans,
                                        ctx.out_dtype, g.value, ctx.num_cu)
-        grad_b = grouped_gemm_fp8_variable_k_impl(a8, qg.qdata, sa, qg.scale_inv, group_lens, group_offs, True,
+        grad_b = grouped_gemm_fp8_variable_k_impl(a8, qg, sa, sg, group_lens, group_offs, True,
                                                   False, ctx.trans_b, ctx.out_dtype, g.value, ctx.num_cu)
-        return grad_a, grad_b, None, None, None, None, None, None, None, None
+        return grad_a, grad_b, None, None, None, None, None, None, None, None, None
 
 
 class FP8GroupedGemmMXFunc(torch.autograd.Function):
@@ -269,8 +274,11 @@ def grouped_gemm_fp8(
     if out_dtype is None:
         out_dtype = torch.promote_types(a_data.dtype, b_data.dtype)
     if config.granularity == ScalingGranularity.TENSORWISE:
+        # a call that no gradient can follow makes no transposed weight
+        need_bwd = torch.is_grad_enabled() and any(
+            t is not None and t.requires_grad for t in (a_data, b_data, a_data_t, b_data_t))
         return FP8GroupedGemmTensorFunc.apply(a_data, b_data, a_data_t, b_data_t, group_lens, group_offs, trans_b,
-                                              out_dtype, config, num_cu)
+                                              out_dtype, config, num_cu, need_bwd)
     elif config.granularity == ScalingGranularity.ROWWISE:
         return FP8GroupedGemmRowFunc.apply(a_data, b_data, a_data_t, b_data_t, group_lens, group_offs, trans_b,
                                            out_dtype, config, num_cu)

@@ -32,3 +32,31 @@ def test_large_tile_loop_edges(scales, K, mn):
     torch.cuda.synchronize()
     assert torch.equal(large.view(torch.int16), small.view(torch.int16))
     assert torch.equal(large.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("gran", ["TENSORWISE", "ROWWISE", "BLOCKWISE", "MX_BLOCKWISE"])
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("mnk", [(33, 264, 160), (256, 512, 384)])
+def test_forward_without_gradients_is_the_same(gran, trans_b, mnk):
+    """A call that no gradient can follow makes no backward copies: the same
+    output, for high-precision operands and for a weight quantized once."""
+    import primus_turbo.pytorch as turbo
+    from primus_turbo.pytorch.core.low_precision import Float8QuantConfig, ScaleDtype, ScalingGranularity
+    from primus_turbo.pytorch.core.quantized_tensor import QuantizedTensor, create_quantized_weight
+
+    if gran == "MX_BLOCKWISE" and not trans_b:
+        pytest.skip("MX takes the NT layout")
+    more = {"BLOCKWISE": dict(block_size=128), "MX_BLOCKWISE": dict(block_size=32, scale_dtype=ScaleDtype.E8M0)}
+    cfg = Float8QuantConfig(granularity=ScalingGranularity[gran], **more.get(gran, {}))
+    M, N, K = mnk
+    g = torch.Generator().manual_seed(5)
+    a = torch.randn((M, K), generator=g).bfloat16().cuda()
+    w = torch.randn((N, K) if trans_b else (K, N), generator=g).bfloat16().cuda()
+    want = turbo.ops.gemm_fp8(a.clone().requires_grad_(), w, trans_b=trans_b, config=cfg)
+    with torch.no_grad():
+        assert torch.equal(turbo.ops.gemm_fp8(a, w, trans_b=trans_b, config=cfg), want)
+    assert torch.equal(turbo.ops.gemm_fp8(a, w, trans_b=trans_b, config=cfg), want)
+    if trans_b or gran in ("TENSORWISE", "BLOCKWISE"):
+        qw = create_quantized_weight(w, torch.float8_e4m3fn, cfg)[0]
+        assert isinstance(qw, QuantizedTensor)
+        assert torch.equal(turbo.ops.gemm_fp8(a, qw, trans_b=trans_b, config=cfg), want)
