@@ -33,25 +33,51 @@
 #ifndef PTA_SPLIT_MIN_K_QUARTER
 #define PTA_SPLIT_MIN_K_QUARTER 3072
 #endif
+#ifndef PTA_SPLIT_MIN_K_1D_1D
+#define PTA_SPLIT_MIN_K_1D_1D 2048
+#endif
 
 namespace pta {
 using namespace gemm_detail;
 
 // K split for problems of at most half a round of tiles (one 256 x 256 tile
-// per CU and round) and K >= 4096, or at most a quarter round and K >= 3072:
-// every tile runs as two half-K workgroups whose fp32 partials meet in the
-// workspace, so twice as many CUs work.  The hand-over (256 KB written and
+// per CU and round) and 32 K blocks or more, or at most a quarter round and 24 K
+// blocks: every tile runs as two half-K workgroups whose fp32 partials meet in
+// the workspace, so twice as many CUs work.  The hand-over (256 KB written and
 // read per tile) costs a fixed ~6-10 us, so a shorter K runs whole
 // (kernel-trace medians, split / whole; 108 tiles: K = 2048 1.22-1.27, 3072
 // 1.01-1.04, 4096 0.92-0.98, 6144 0.78-0.80; 128 tiles: 2048 1.14-1.22, 3072
-// 0.99-1.00; 64 tiles: 2048 1.02-1.03, 3072 0.84, 4096 0.78-0.81).  Splitting
+// 0.99-1.00; 64 tiles: 2048 1.02-1.03, 3072 0.84, 4096 0.78-0.81).  With 1-D
+// scales on both operands a K block takes longer, and up to 3/8 of a round
+// splits from 16 K blocks (K = 2048: 64 tiles 32.7 -> 28.8 us, 96 tiles 32.8 ->
+// 30.2, 128 tiles 33.2 both).  A K that is no multiple of 128 splits by the same
+// rule (K = 4000: blockwise 52 tiles 49.1 -> 38.9 us, 64 45.6 -> 35.0, 96 46.0 ->
+// 37.1, 128 46.7 -> 43.6; 1-D by 1-D 57.9 -> 41.1 at 64), except for tensorwise /
+// rowwise scales past 3/8 of a round (128 tiles: 41.3 -> 42.7).  Splitting
 // the last round of larger problems measured no faster (headline
 // 4096x18432x7168: +1%), so those run whole.  Returns the number of split
 // tiles (0: none).
-int64_t split_tiles(int64_t tiles, int64_t K, int cus) {
-    if (K % BK != 0 || tiles <= 0 || cus <= 0 || 2 * tiles > cus) return 0;
-    const int64_t kmin = 4 * tiles <= cus ? PTA_SPLIT_MIN_K_QUARTER : PTA_SPLIT_MIN_K;
-    return K >= kmin ? tiles : 0;
+enum : int { SPLIT_PLAIN = 0, SPLIT_SCALED = 1, SPLIT_1D_1D = 2 }; // tensorwise / rowwise; blockwise or MX; 1-D by 1-D
+
+int64_t split_tiles(int64_t tiles, int64_t K, int cus, int kind) {
+    if (tiles <= 0 || cus <= 0 || 2 * tiles > cus) return 0;
+    const bool three8 = 8 * tiles <= 3 * static_cast<int64_t>(cus);
+    if (K % BK != 0 && kind == SPLIT_PLAIN && !three8) return 0;
+    int64_t kmin = 4 * tiles <= cus ? PTA_SPLIT_MIN_K_QUARTER : PTA_SPLIT_MIN_K;
+    if (kind == SPLIT_1D_1D && three8) kmin = PTA_SPLIT_MIN_K_1D_1D;
+    return cdiv(K, BK) * BK >= kmin ? tiles : 0;
+}
+
+// the same for any kind of scales (workspace sizes)
+int64_t split_tiles_most(int64_t tiles, int64_t K, int cus) {
+    int64_t n = 0;
+    for (int k = SPLIT_PLAIN; k <= SPLIT_1D_1D; ++k) n = n > split_tiles(tiles, K, cus, k) ? n : split_tiles(tiles, K, cus, k);
+    return n;
+}
+
+int split_kind(int sm, bool a2d, bool b2d) {
+    if (sm == SM_TENSOR || sm == SM_ROW) return SPLIT_PLAIN;
+    return sm == SM_BLOCK && !a2d && !b2d ? SPLIT_1D_1D : SPLIT_SCALED;
 }
 
 constexpr int64_t SPLIT_TILE_BYTES = int64_t(BM) * BN * 4;
@@ -85,7 +111,7 @@ int gemm_nt_launch(const uint8_t *a, int fa, int64_t lda, const uint8_t *b, int 
     g.aligned_c = ((ldc * (out_dt == PTA_F32 ? 4 : 2)) % 16 == 0) && aligned16(c);
     if (split_ws != nullptr && !stream_capturing(st)) {
         // a graph would replay the call tag, so captured calls do not split
-        const int64_t ns = split_tiles(int64_t(g.tiles_m) * g.tiles_n, K, device_cu_count());
+        const int64_t ns = split_tiles(int64_t(g.tiles_m) * g.tiles_n, K, device_cu_count(), split_kind(sm, a2d, b2d));
         if (ns > 0) {
             const uint64_t tag = next_call_tag();
             const WaitPlan w   = wait_plan(tag, SPLIT_SPIN_LIMIT);
@@ -227,7 +253,7 @@ static bool small_path(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b
     // K-contiguous operands, a quarter of a round of 256 x 256 tiles or more
     // and a long K: the large tiles with the K split are faster (blockwise
     // 1024x4096x4096: 62 -> 45 us; at K = 2048 or with fewer tiles they are not)
-    if (!kmajor && tiles >= 48 && K >= 4096 && K % 128 == 0) return false;
+    if (!kmajor && tiles >= 48 && cdiv(K, 128) >= 32) return false;
     if (!kmajor && block_on_128_tiles(M, N, sm)) return false;
     const int64_t lim = int64_t(1) << 30;
     if (trans_a ? (M % 8 != 0 || (K + 1024) * M >= lim) : 64 * K >= lim) return false;
@@ -241,7 +267,7 @@ extern "C" size_t pta_gemm_fp8_workspace_size(int64_t M, int64_t N, int64_t K, i
     size_t ws = 0;
     if (trans_a) ws += static_cast<size_t>(cdiv(M * K, 256) * 256);
     if (!trans_b) ws += static_cast<size_t>(cdiv(N * K, 256) * 256);
-    ws += static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
+    ws += static_cast<size_t>(split_ws_bytes(split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
     return ws;
 }
 
@@ -294,7 +320,7 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
         wsp += cdiv(N * K, 256) * 256;
     }
     // what remains of the workspace holds the K split's partial tiles
-    uint8_t      *split_ws  = split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count()) > 0 ? wsp : nullptr;
+    uint8_t      *split_ws  = split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count()) > 0 ? wsp : nullptr;
     const int64_t split_off = workspace != nullptr ? wsp - static_cast<uint8_t *>(workspace) : 0;
     // scale strides in the NT view
     bool    a2d = false, b2d = false;
@@ -334,7 +360,7 @@ static bool strided_small_path(int64_t M, int64_t N, int64_t K, int64_t lda, int
                                int64_t sb_bytes, int sm) {
     const int64_t tiles = cdiv(M, BM) * cdiv(N, BN);
     if (tiles >= PTA_SMALL_MAX_TILES) return false;
-    if (tiles >= 48 && K >= 4096 && K % 128 == 0) return false; // the K split is faster there
+    if (tiles >= 48 && cdiv(K, 128) >= 32) return false; // the K split is faster there
     if (block_on_128_tiles(M, N, sm)) return false;
     const int64_t lim = int64_t(1) << 30;
     return 64 * lda < lim && 64 * ldb < lim && sa_bytes < 2 * lim && sb_bytes < 2 * lim;
@@ -343,7 +369,7 @@ static bool strided_small_path(int64_t M, int64_t N, int64_t K, int64_t lda, int
 static size_t strided_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t sa_bytes,
                                int64_t sb_bytes, int sm) {
     if (strided_small_path(M, N, K, lda, ldb, sa_bytes, sb_bytes, sm)) return 0;
-    return static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
+    return static_cast<size_t>(split_ws_bytes(split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
 }
 
 // choose: pick the small-tile kernel or the K split as pta_gemm_fp8 does

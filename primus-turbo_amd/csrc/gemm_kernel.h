@@ -400,8 +400,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
             C       = reinterpret_cast<uint8_t *>(g.c) + q * g.c_gstride;
         }
         if (split_half >= 0) {
-            // K % BK == 0 here; the second half starts at K block nk / 2
-            const int64_t kh = (K / BK) / 2;
+            // the second half starts at K block nk / 2 (and has the cut last block)
+            const int64_t kh = ((K + BK - 1) / BK) / 2;
             if (split_half == 0) {
                 K = kh * BK;
             } else {
