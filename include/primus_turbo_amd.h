@@ -145,6 +145,7 @@ int pta_quantize_fp8_blockwise(const void *x, int in_dtype, int64_t M, int64_t N
 /* Layout flags of pta_quantize_fp8_blockwise_dual. */
 #define PTA_DUAL_COL_TRANSPOSED 1   /* q_col written as [N, roundup(M, 128)], zero padded */
 #define PTA_DUAL_ROW_SCALE_KMAJOR 2 /* s_row written as [ceil(N/block), M] */
+#define PTA_DUAL_ROW_PAD16 4        /* q_row written as [M, roundup(N, 16)], zero padded */
 
 /* Blockwise dual (one read of x): row-scaled q_row[M,N] + s_row[M, ceil(N/block)]
  * and col-scaled q_col + s_col[ceil(M/block), N].  Without flags q_col is
@@ -153,7 +154,8 @@ int pta_quantize_fp8_blockwise(const void *x, int in_dtype, int64_t M, int64_t N
  * zero padded (K-contiguous operand for the NT wgrad GEMM);
  * PTA_DUAL_ROW_SCALE_KMAJOR stores s_row(m, kb) at s_row[kb * M + m], so a GEMM
  * reading the scales of one K block for consecutive rows touches consecutive
- * words.  Either output pair may be NULL.
+ * words; PTA_DUAL_ROW_PAD16 pads q_row's rows to the 16-byte multiple that the
+ * GEMM entries take.  Either output pair may be NULL.
  * Replaces quant_fp8_blockwise_dual_impl (quantization_impl.py:229-274). */
 int pta_quantize_fp8_blockwise_dual(const void *x, int in_dtype, int64_t M, int64_t N,
                                     int64_t block, void *q_row, float *s_row, void *q_col,
@@ -167,6 +169,12 @@ int pta_quantize_fp8_blockwise_dual(const void *x, int in_dtype, int64_t M, int6
 int pta_quantize_fp8_blockwise_for_weight(const void *w, int in_dtype, int64_t B, int64_t M,
                                           int64_t N, int64_t block, void *q, float *s, void *q_t,
                                           int fmt, pta_stream_t stream);
+
+/* The same with q written as [B, M, roundup(N, 16)], zero padded (rows that the
+ * GEMM entries take for any N). */
+int pta_quantize_fp8_blockwise_for_weight_pad16(const void *w, int in_dtype, int64_t B, int64_t M,
+                                                int64_t N, int64_t block, void *q, float *s, void *q_t,
+                                                int fmt, pta_stream_t stream);
 
 /* layout flag of pta_quantize_fp8_blockwise_segment_m_row_col: q_col_pad is
  * written transposed, [N, roundup(M, 128) + 128 * G] (column m = padded row m,

@@ -40,6 +40,7 @@ struct QBArgs {
     int64_t     M, N;      // input rows / cols (per batch for W2D)
     int64_t     batch_stride_x;
     uint8_t    *q_row;     // ROW / W2D output
+    int64_t     ldr;       // its row stride: N, or N rounded up to 16 (pad bytes are written as zero)
     float      *s_row;     // ROW: s_row[r * srow_m + kb * srow_k]
     int64_t     srow_m, srow_k;
     uint8_t    *q_col;     // COL output
@@ -126,13 +127,33 @@ __device__ __forceinline__ void st16(void *dst, uint32_t a, uint32_t b, uint32_t
     else *reinterpret_cast<v4u *>(dst) = v;
 }
 
+// 16 fp8 bytes of a row at dst, `left` of them inside the row (rows of `ld` bytes)
+template <int VEC, bool NT_STORE>
+__device__ __forceinline__ void st_segment(uint8_t *dst, const uint32_t (&w)[4], int64_t left, int64_t ld) {
+    if (VEC == 2 || (VEC == 1 && ld % 16 == 0)) {
+        if (left >= 16) st16<NT_STORE>(dst, w[0], w[1], w[2], w[3]);
+    } else if (VEC == 1) {
+        if (left >= 8) *reinterpret_cast<uint2 *>(dst) = make_uint2(w[0], w[1]);
+        if (left >= 16) *reinterpret_cast<uint2 *>(dst + 8) = make_uint2(w[2], w[3]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (j < left) dst[j] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
+    }
+}
+
 // STREAM: 0 plain accesses, 1 non-temporal input loads, 2 non-temporal output stores (plain loads).
+// VEC: 2 16-byte loads and stores (rows of whole 16-element segments); 1 rows of
+// whole 8-element chunks: 16-byte loads, guarded per chunk, and 8-byte stores, or
+// 16-byte ones into padded rows (4000 x 3080 weight with transposed copy 11.6 us
+// against 42 element by element, 1000 x 3080 dual 9.2 against 18); 0 element by
+// element.
 // TPW: tiles per workgroup.  With 2, the workgroup's two halves (256 lanes
 // each) take two neighbouring tiles of one tile row (row-major order) or one
 // tile column (column-major order), so the workgroup reads 512-byte row
 // segments; both halves run the same barriers (the tile-dependent branch of
 // the weight mode is taken by both when either tile needs it).
-template <int IN_DT, int FMT, int MODE, bool VEC, int STREAM, int TPW>
+template <int IN_DT, int FMT, int MODE, int VEC, int STREAM, int TPW>
 __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args) {
     const int     half  = TPW == 2 ? static_cast<int>(threadIdx.x >> 8) : 0;
     const int     t     = static_cast<int>(threadIdx.x) & (NT - 1);
@@ -204,18 +225,18 @@ __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args)
     for (int i = 0; i < 4; ++i) {
         const int64_t r = row_base + rgrp * 4 + i;
         rvalid[i]       = (r >= row_lo) && (r < row_hi);
-        if (VEC) {
+        if constexpr (VEC > 0) {
             // conditional global loads.  (Loads through a buffer resource that
             // spans the tile's valid rows, out-of-range rows reading as zero,
             // issue all eight back to back with no branches, and measured 1-3%
             // slower on the large streamed tensors, no faster on the rest.)
             typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-            const bool   ok = rvalid[i] && n0 + 16 <= N;
+            constexpr int CE = 16 / CH; // elements per 16-byte chunk
             const v4u   *p  = reinterpret_cast<const v4u *>(xb + (r * N + n0) * InTraits<IN_DT>::bytes);
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
                 v4u w = v4u{0u, 0u, 0u, 0u};
-                if (ok) {
+                if (rvalid[i] && n0 + (VEC == 2 ? 16 : CE * (c + 1)) <= N) {
                     if constexpr (STREAM == 1) w = __builtin_nontemporal_load(p + c);
                     else w = p[c];
                 }
@@ -333,14 +354,7 @@ __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args)
 #pragma unroll
                     for (int k = 0; k < 4; ++k) w[k] = F4(i, 4 * k, sc[i]);
                 }
-                uint8_t *dst = args.q_row + r * N + n0;
-                if (VEC && n0 + 16 <= N) {
-                    st16<(STREAM == 2)>(dst, w[0], w[1], w[2], w[3]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (n0 + j < N) dst[j] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
-                }
+                st_segment<VEC, (STREAM == 2)>(args.q_row + r * args.ldr + n0, w, args.ldr - n0, args.ldr);
             }
         }
     }
@@ -402,14 +416,7 @@ __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args)
                         w[k] = cast4<FMT>(V(i, 4 * k) * cs[4 * k], V(i, 4 * k + 1) * cs[4 * k + 1],
                                           V(i, 4 * k + 2) * cs[4 * k + 2], V(i, 4 * k + 3) * cs[4 * k + 3]);
                 }
-                uint8_t *dst = args.q_col + prow * N + n0;
-                if (VEC && n0 + 16 <= N) {
-                    st16<(STREAM == 2)>(dst, w[0], w[1], w[2], w[3]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (n0 + j < N) dst[j] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
-                }
+                st_segment<VEC, (STREAM == 2)>(args.q_col + prow * N + n0, w, N - n0, N);
             }
         } else {
             // transposed output q_col[N, M]: stage bytes column-major in LDS
@@ -475,7 +482,7 @@ __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args)
         const float   sc  = scale_from_amax<FMT>(a, 1e-4f);
         const int64_t mb  = (M + TILE - 1) / TILE, nb = (N + TILE - 1) / TILE;
         if (t == 0) args.s_w[(batch * mb + tm) * nb + tn] = 1.0f / sc;
-        uint8_t *qb = args.q_row + batch * M * N;
+        uint8_t *qb = args.q_row + batch * M * args.ldr;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int64_t r = row_base + rgrp * 4 + i;
@@ -488,14 +495,7 @@ __global__ __launch_bounds__(NT * TPW) void quant_block_tile_kernel(QBArgs args)
                 for (int k = 0; k < 4; ++k) w[k] = F4(i, 4 * k, sc);
             }
             if (!rvalid[i]) continue;
-            uint8_t *dst = qb + r * N + n0;
-            if (VEC && n0 + 16 <= N) {
-                st16<(STREAM == 2)>(dst, w[0], w[1], w[2], w[3]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    if (n0 + j < N) dst[j] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
-            }
+            st_segment<VEC, (STREAM == 2)>(qb + r * args.ldr + n0, w, args.ldr - n0, args.ldr);
         }
         if constexpr ((MODE & QB_W2D_T) != 0) {
             // transposed copy [B, N, M] through LDS.  The bytes are quantized
@@ -608,14 +608,14 @@ uint32_t tile_grid(int64_t rows, int64_t cols) {
 }
 
 template <int MODE>
-int launch_tile(const QBArgs &a, int in_dtype, int fmt, dim3 grid, bool vec, hipStream_t st) {
+int launch_tile(const QBArgs &a, int in_dtype, int fmt, dim3 grid, int vec, hipStream_t st) {
     PTA_CHECK_ARG(grid.x <= 0x7fffffffu, "tensor too large: more than 2^31 - 1 tiles of 128 x 128");
     if (grid.x == 0) return PTA_OK;
     const int64_t elems    = static_cast<int64_t>(grid.z) * a.M * a.N;
     const int64_t in_bytes = elems * (in_dtype == PTA_F32 ? 4 : 2);
     // fp8 byte outputs written by this mode
     const int64_t nq        = ((MODE & (QB_ROW | QB_W2D)) ? 1 : 0) + ((MODE & QB_COL) ? 1 : 0) + ((MODE & QB_W2D_T) ? 1 : 0);
-    const bool    stream    = vec && in_bytes >= STREAM_BYTES;
+    const bool    stream    = vec == 2 && in_bytes >= STREAM_BYTES;
     const bool    nt_store  = stream && elems * nq >= NT_STORE_BYTES;
     // the load hint for the 1-D modes whose outputs fit the MALL (row-only / column-only
     // 28672 x 8192: 1.6% / 2.2% faster); the 128 x 128 weight mode reads faster without it
@@ -628,7 +628,7 @@ int launch_tile(const QBArgs &a, int in_dtype, int fmt, dim3 grid, bool vec, hip
     const dim3     grid2(grid.x / 2, grid.y, grid.z);
 #define PTA_QB_LAUNCH(IDT, F, V, S)                                                                \
     do {                                                                                           \
-        if constexpr (V) {                                                                         \
+        if constexpr (V == 2) {                                                                    \
             if (pair) {                                                                            \
                 quant_block_tile_kernel<IDT, F, MODE, V, S, 2><<<grid2, 2 * NT, 0, st>>>(a);       \
                 break;                                                                             \
@@ -640,10 +640,11 @@ int launch_tile(const QBArgs &a, int in_dtype, int fmt, dim3 grid, bool vec, hip
     if (fmt == PTA_E4M3) PTA_QB_LAUNCH(IDT, PTA_E4M3, V, S);                                       \
     else PTA_QB_LAUNCH(IDT, PTA_E5M2, V, S)
 #define PTA_QB_VEC(IDT)                                                                            \
-    if (nt_store) { PTA_QB_FMT(IDT, true, 2); }                                                    \
-    else if (nt_load) { PTA_QB_FMT(IDT, true, 1); }                                                \
-    else if (vec) { PTA_QB_FMT(IDT, true, 0); }                                                    \
-    else { PTA_QB_FMT(IDT, false, 0); }
+    if (nt_store) { PTA_QB_FMT(IDT, 2, 2); }                                                       \
+    else if (nt_load) { PTA_QB_FMT(IDT, 2, 1); }                                                   \
+    else if (vec == 2) { PTA_QB_FMT(IDT, 2, 0); }                                                  \
+    else if (vec == 1) { PTA_QB_FMT(IDT, 1, 0); }                                                  \
+    else { PTA_QB_FMT(IDT, 0, 0); }
     if (in_dtype == PTA_BF16) { PTA_QB_VEC(PTA_BF16) }
     else if (in_dtype == PTA_F16) { PTA_QB_VEC(PTA_F16) }
     else { PTA_QB_VEC(PTA_F32) }
@@ -654,13 +655,17 @@ int launch_tile(const QBArgs &a, int in_dtype, int fmt, dim3 grid, bool vec, hip
     return PTA_OK;
 }
 
-bool vec_ok(const void *x, int in_dtype, int64_t N, std::initializer_list<const void *> outs) {
+// access width of the kernel (its VEC): rows of whole 16-element segments, of
+// whole 8-element chunks, or neither; everything aligned
+int vec_ok(const void *x, int in_dtype, int64_t N, std::initializer_list<const void *> outs) {
     const int64_t eb = in_dtype == PTA_F32 ? 4 : 2;
-    if (!aligned16(x) || (N * eb) % 16 != 0 || N % 16 != 0) return false;
+    if (!aligned16(x) || (N * eb) % 16 != 0 || N % 8 != 0) return 0;
     for (const void *p : outs)
-        if (p && !aligned16(p)) return false;
-    return true;
+        if (p && !aligned16(p)) return 0;
+    return N % 16 == 0 ? 2 : 1;
 }
+
+int64_t row_stride16(int64_t N) { return cdiv(N, 16) * 16; }
 
 int check_common(const void *x, int in_dtype, int fmt, int64_t block) {
     PTA_CHECK_ARG(x != nullptr, "input pointer is NULL");
@@ -686,9 +691,9 @@ extern "C" int pta_quantize_fp8_blockwise(const void *x, int in_dtype, int64_t M
     PTA_CHECK_ARG(axis == 0 || axis == 1, "axis must be 0 or 1");
     if (M == 0 || N == 0) return PTA_OK;
     QBArgs a{};
-    a.x = x; a.M = M; a.N = N;
+    a.x = x; a.M = M; a.N = N; a.ldr = N;
     dim3 grid(tile_grid(M, N), 1, 1);
-    const bool v = vec_ok(x, in_dtype, N, {q});
+    const int v = vec_ok(x, in_dtype, N, {q});
     if (axis == 1) {
         a.q_row = static_cast<uint8_t *>(q); a.s_row = s;
         a.srow_m = cdiv(N, TILE); a.srow_k = 1;
@@ -708,19 +713,21 @@ extern "C" int pta_quantize_fp8_blockwise_dual(const void *x, int in_dtype, int6
     PTA_CHECK_ARG((q_row == nullptr) == (s_row == nullptr), "q_row/s_row must both be set or NULL");
     PTA_CHECK_ARG((q_col == nullptr) == (s_col == nullptr), "q_col/s_col must both be set or NULL");
     PTA_CHECK_ARG(q_row || q_col, "no output requested");
-    PTA_CHECK_ARG((layout & ~(PTA_DUAL_COL_TRANSPOSED | PTA_DUAL_ROW_SCALE_KMAJOR)) == 0, "unknown layout flags");
+    PTA_CHECK_ARG((layout & ~(PTA_DUAL_COL_TRANSPOSED | PTA_DUAL_ROW_SCALE_KMAJOR | PTA_DUAL_ROW_PAD16)) == 0,
+                  "unknown layout flags");
     if (M == 0 || N == 0) return PTA_OK;
     const bool col_transposed = (layout & PTA_DUAL_COL_TRANSPOSED) != 0;
     QBArgs     a{};
-    a.x = x; a.M = M; a.N = N;
+    a.x = x; a.M = M; a.N = N; a.ldr = N;
     a.q_row = static_cast<uint8_t *>(q_row); a.s_row = s_row;
+    if (layout & PTA_DUAL_ROW_PAD16) a.ldr = row_stride16(N);
     if (layout & PTA_DUAL_ROW_SCALE_KMAJOR) { a.srow_m = 1; a.srow_k = M; }
     else { a.srow_m = cdiv(N, TILE); a.srow_k = 1; }
     a.q_col = static_cast<uint8_t *>(q_col); a.s_col = s_col;
     a.ldt_col = cdiv(M, TILE) * TILE;
     dim3       grid(tile_grid(M, N), 1, 1);
     PTA_CHECK_ARG(!col_transposed || aligned16(q_col), "transposed q_col must be 16-byte aligned");
-    const bool v = vec_ok(x, in_dtype, N, {q_row, col_transposed ? nullptr : q_col});
+    const int v = vec_ok(x, in_dtype, N, {q_row, col_transposed ? nullptr : q_col});
     hipStream_t st = as_stream(stream);
     if (q_row && q_col) {
         return col_transposed ? launch_tile<QB_ROW | QB_COL | QB_COL_T>(a, in_dtype, fmt, grid, v, st)
@@ -731,10 +738,8 @@ extern "C" int pta_quantize_fp8_blockwise_dual(const void *x, int in_dtype, int6
                           : launch_tile<QB_COL>(a, in_dtype, fmt, grid, v, st);
 }
 
-extern "C" int pta_quantize_fp8_blockwise_for_weight(const void *w, int in_dtype, int64_t B,
-                                                     int64_t M, int64_t N, int64_t block, void *q,
-                                                     float *s, void *q_t, int fmt,
-                                                     pta_stream_t stream) {
+static int quantize_weight(const void *w, int in_dtype, int64_t B, int64_t M, int64_t N, int64_t block, void *q,
+                           int64_t ldq, float *s, void *q_t, int fmt, pta_stream_t stream) {
     clear_error();
     if (int rc = check_common(w, in_dtype, fmt, block)) return rc;
     PTA_CHECK_ARG(B >= 0 && M >= 0 && N >= 0, "negative shape");
@@ -742,14 +747,28 @@ extern "C" int pta_quantize_fp8_blockwise_for_weight(const void *w, int in_dtype
     if (B == 0 || M == 0 || N == 0) return PTA_OK;
     PTA_CHECK_ARG(B <= 65535, "batch too large");
     QBArgs a{};
-    a.x = w; a.M = M; a.N = N; a.batch_stride_x = M * N;
+    a.x = w; a.M = M; a.N = N; a.ldr = ldq; a.batch_stride_x = M * N;
     a.q_row = static_cast<uint8_t *>(q); a.s_w = s; a.q_t = static_cast<uint8_t *>(q_t);
     dim3 grid(tile_grid(M, N), 1, static_cast<uint32_t>(B));
     PTA_CHECK_ARG(!q_t || aligned16(q_t), "q_t must be 16-byte aligned");
-    const bool v = vec_ok(w, in_dtype, N, {q}) && (M * N * (in_dtype == PTA_F32 ? 4 : 2)) % 16 == 0;
+    const int v = (M * N * (in_dtype == PTA_F32 ? 4 : 2)) % 16 == 0 ? vec_ok(w, in_dtype, N, {q}) : 0;
     hipStream_t st = as_stream(stream);
     if (q_t) return launch_tile<QB_W2D | QB_W2D_T>(a, in_dtype, fmt, grid, v, st);
     return launch_tile<QB_W2D>(a, in_dtype, fmt, grid, v, st);
+}
+
+extern "C" int pta_quantize_fp8_blockwise_for_weight(const void *w, int in_dtype, int64_t B,
+                                                     int64_t M, int64_t N, int64_t block, void *q,
+                                                     float *s, void *q_t, int fmt,
+                                                     pta_stream_t stream) {
+    return quantize_weight(w, in_dtype, B, M, N, block, q, N, s, q_t, fmt, stream);
+}
+
+extern "C" int pta_quantize_fp8_blockwise_for_weight_pad16(const void *w, int in_dtype, int64_t B,
+                                                           int64_t M, int64_t N, int64_t block, void *q,
+                                                           float *s, void *q_t, int fmt,
+                                                           pta_stream_t stream) {
+    return quantize_weight(w, in_dtype, B, M, N, block, q, row_stride16(N), s, q_t, fmt, stream);
 }
 
 extern "C" int pta_quantize_fp8_blockwise_segment_m_row_col(
@@ -768,7 +787,7 @@ extern "C" int pta_quantize_fp8_blockwise_segment_m_row_col(
     if (N == 0) return PTA_OK;
     const int64_t M_pad_max = M + G * TILE;
     QBArgs        a{};
-    a.x = x; a.M = M; a.N = N;
+    a.x = x; a.M = M; a.N = N; a.ldr = N;
     a.q_row = static_cast<uint8_t *>(q_row); a.s_row = s_row_t;
     a.srow_m = 1; a.srow_k = M;
     a.q_col = static_cast<uint8_t *>(q_col_pad); a.s_col = s_col_pad;
@@ -779,10 +798,10 @@ extern "C" int pta_quantize_fp8_blockwise_segment_m_row_col(
         // q_col [N, roundup(M, 128) + 128 G]: column m of the transposed copy is
         // row m of the padded layout (16-byte chunks, zero padding rows)
         PTA_CHECK_ARG(aligned16(q_col_pad), "transposed q_col must be 16-byte aligned");
-        const bool v = vec_ok(x, in_dtype, N, {q_row});
+        const int v = vec_ok(x, in_dtype, N, {q_row});
         return launch_tile<QB_ROW | QB_COL | QB_COL_T | QB_SEGMENT>(a, in_dtype, fmt, grid, v, st);
     }
-    const bool v = vec_ok(x, in_dtype, N, {q_row, q_col_pad});
+    const int v = vec_ok(x, in_dtype, N, {q_row, q_col_pad});
     return launch_tile<QB_ROW | QB_COL | QB_SEGMENT>(a, in_dtype, fmt, grid, v, st);
 }
 

@@ -18,7 +18,7 @@ PTA_F32, PTA_F16, PTA_BF16 = 0, 1, 2
 PTA_E4M3, PTA_E5M2 = 0, 1
 PTA_TENSORWISE, PTA_ROWWISE, PTA_BLOCKWISE, PTA_MX_BLOCKWISE = 1, 2, 3, 4
 # layout flags of pta_quantize_fp8_blockwise_dual
-DUAL_COL_TRANSPOSED, DUAL_ROW_SCALE_KMAJOR = 1, 2
+DUAL_COL_TRANSPOSED, DUAL_ROW_SCALE_KMAJOR, DUAL_ROW_PAD16 = 1, 2, 4
 # exponent layout flag of pta_quantize_mxfp8
 MX_EXP_KMAJOR = 1
 # layout flag of pta_quantize_fp8_blockwise_segment_m_row_col
@@ -43,6 +43,7 @@ SIGNATURES = {
     "pta_quantize_fp8_blockwise": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _vp, _vp, _i32, _vp]),
     "pta_quantize_fp8_blockwise_dual": (_i32, [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "pta_quantize_fp8_blockwise_for_weight": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp]),
+    "pta_quantize_fp8_blockwise_for_weight_pad16": (_i32, [_vp, _i32, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp]),
     "pta_quantize_fp8_blockwise_segment_m_row_col": (
         _i32,
         [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp],

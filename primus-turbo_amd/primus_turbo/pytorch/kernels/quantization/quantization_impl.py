@@ -168,6 +168,7 @@ def quant_fp8_blockwise_dual_impl(
     col_transposed: bool = False,
     row_scale_kmajor: bool = False,
     row_only: bool = False,
+    row_pad16: bool = False,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """Row (1 x bs) and column (bs x 1) quantization in one read of ``x``.
 
@@ -179,13 +180,14 @@ def quant_fp8_blockwise_dual_impl(
     - ``row_scale_kmajor=True`` returns the row scales as a ``[M, N/bs]`` view
       of ``[N/bs, M]`` storage (strides ``(1, M)``): the GEMM then reads the
       scales of one K block for 16 consecutive rows from one cache line.
-    ``row_only=True`` leaves the column outputs out (None).
+    ``row_only=True`` leaves the column outputs out (None); ``row_pad16=True`` pads
+    q_row's rows with zeros to a multiple of 16 (the GEMM's row granularity).
     """
     _check_hp(x)
     assert x.is_contiguous() and x.dim() == 2, "Input must be 2D and contiguous"
     M, N = x.shape
     nb = ceil_div(N, block_size)
-    q_row = torch.empty((M, N), dtype=dtype, device=x.device)
+    q_row = torch.empty((M, ceil_div(N, 16) * 16 if row_pad16 else N), dtype=dtype, device=x.device)
     if row_scale_kmajor:
         s_row = torch.empty((nb, M), dtype=torch.float32, device=x.device).t()
     else:
@@ -195,6 +197,7 @@ def quant_fp8_blockwise_dual_impl(
         q_col = torch.empty((N, ceil_div(M, 128) * 128) if col_transposed else (M, N), dtype=dtype, device=x.device)
         s_col = torch.empty((ceil_div(M, block_size), N), dtype=torch.float32, device=x.device)
     layout = (_C.DUAL_COL_TRANSPOSED if col_transposed else 0) | (_C.DUAL_ROW_SCALE_KMAJOR if row_scale_kmajor else 0)
+    layout |= _C.DUAL_ROW_PAD16 if row_pad16 else 0
     _C.call(
         "pta_quantize_fp8_blockwise_dual", _C.ptr(x), _C.in_dtype_code(x.dtype), M, N, block_size, _C.ptr(q_row),
         _C.ptr(s_row), _C.ptr(q_col), _C.ptr(s_col), layout, _C.fp8_code(dtype), _C.stream(x.device),
@@ -203,20 +206,21 @@ def quant_fp8_blockwise_dual_impl(
 
 
 def quant_fp8_blockwise_for_weight_impl(
-    w: torch.Tensor, dtype: torch.dtype, block_size: int = 128, with_transpose: bool = False
+    w: torch.Tensor, dtype: torch.dtype, block_size: int = 128, with_transpose: bool = False, pad16: bool = False
 ):
     """128 x 128 weight blocks; returns (q, s) or (q, s, q_t) with ``with_transpose``
-    (q_t: the same bytes as [B, N, roundup(M, 128)], zero padded)."""
+    (q_t: the same bytes as [B, N, roundup(M, 128)], zero padded).  ``pad16=True``
+    pads q's rows with zeros to a multiple of 16."""
     _check_hp(w)
     assert w.dim() in (2, 3)
     w = w.contiguous()
     squeeze = w.dim() == 2
     B, M, N = (1, *w.shape) if squeeze else tuple(w.shape)
-    q = torch.empty((B, M, N), dtype=dtype, device=w.device)
+    q = torch.empty((B, M, ceil_div(N, 16) * 16 if pad16 else N), dtype=dtype, device=w.device)
     s = torch.empty((B, ceil_div(M, block_size), ceil_div(N, block_size)), dtype=torch.float32, device=w.device)
     q_t = torch.empty((B, N, ceil_div(M, 128) * 128), dtype=dtype, device=w.device) if with_transpose else None
     _C.call(
-        "pta_quantize_fp8_blockwise_for_weight", _C.ptr(w), _C.in_dtype_code(w.dtype), B, M, N, block_size,
+        "pta_quantize_fp8_blockwise_for_weight_pad16" if pad16 else "pta_quantize_fp8_blockwise_for_weight", _C.ptr(w), _C.in_dtype_code(w.dtype), B, M, N, block_size,
         _C.ptr(q), _C.ptr(s), _C.ptr(q_t), _C.fp8_code(dtype), _C.stream(w.device),
     )
     if squeeze:

@@ -265,7 +265,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         else:
             a_row, a_row_s, a_colT, a_col_s = quant_fp8_blockwise_dual_impl(
                 a.detach().contiguous(), fdt, block_size=config.block_size, col_transposed=True,
-                row_scale_kmajor=True, row_only=not need_bwd,
+                row_scale_kmajor=True, row_only=not need_bwd, row_pad16=True,
             )
         # --- B: 128 x 128 blocks, reused by fwd and dgrad
         recipe = ScalingRecipe(use_2d_block=True)
@@ -275,11 +275,12 @@ class FP8GemmBlockFunction(torch.autograd.Function):
             w_s = b.scale_inv
         elif need_bwd or not trans_b:
             qw, w_s, qw_t = quant_fp8_blockwise_for_weight_impl(
-                b.detach().contiguous(), fdt, block_size=config.block_size, with_transpose=True
+                b.detach().contiguous(), fdt, block_size=config.block_size, with_transpose=True, pad16=True
             )
             w_nk, w_kn = (qw, qw_t) if trans_b else (qw_t, qw)
         else:
-            w_nk, w_s = quant_fp8_blockwise_for_weight_impl(b.detach().contiguous(), fdt, block_size=config.block_size)
+            w_nk, w_s = quant_fp8_blockwise_for_weight_impl(b.detach().contiguous(), fdt, block_size=config.block_size,
+                                                            pad16=True)
         N = w_nk.shape[0]
         a_row = _pad_cols16(a_row)
         w_nk = _pad_cols16(w_nk)
@@ -291,7 +292,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         out = gemm_fp8_nt(a_row, w_nk, out_dtype, gran, a_row_s, a_row_s.stride(), False, w_s, w_str_nk, True)
         if not need_bwd:
             return out
-        ctx.save_for_backward(a_colT, a_col_s, _pad_cols(w_kn, _BLOCK), w_s)
+        ctx.save_for_backward(a_colT, a_col_s, _pad_cols16(w_kn), w_s)
         ctx.w_str_kn = w_str_kn
         ctx.trans_b, ctx.out_dtype, ctx.config = trans_b, out_dtype, config
         ctx.M, ctx.N, ctx.K = M, N, K
@@ -306,7 +307,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         gdt = _get_fp8_dtype(ctx.config.format, False)
         g_row, g_row_s, g_colT, g_col_s = quant_fp8_blockwise_dual_impl(
             grad_out.contiguous(), gdt, block_size=ctx.config.block_size, col_transposed=True,
-            row_scale_kmajor=True,
+            row_scale_kmajor=True, row_pad16=True,
         )
         # dgrad: dA[M, K] = g_row[M, N] . w_kn[K, N]^T
         grad_a = gemm_fp8_nt(_pad_cols16(g_row), w_kn, ctx.out_dtype, gran, g_row_s, g_row_s.stride(), False,
