@@ -499,11 +499,25 @@ __global__ __launch_bounds__(NT) void rw_col_finalize_kernel(const float *partia
     scale_inv[o * inner + n] = 1.0f / sc;
 }
 
+// two fp32 values rounded to 16 bits (to nearest even) and widened again
+template <int DT> __device__ __forceinline__ void round16(float &a, float &b) {
+    if constexpr (DT == PTA_BF16) {
+        typedef float  f2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{a, b}), b2));
+        a = __uint_as_float(w << 16);
+        b = __uint_as_float(w & 0xffff0000u);
+    } else if constexpr (DT == PTA_F16) {
+        a = f16_bits_to_f32(f32_to_f16_bits(a));
+        b = f16_bits_to_f32(f32_to_f16_bits(b));
+    }
+}
+
 // Source of the vector column kernels: 8 consecutive columns of a row as fp32.
 // REQ false: x holds IN_DT elements.  REQ true: x holds fp8 bytes (SFMT) with one
 // scale per row, and an element enters as it would after a dequantization to
-// IN_DT: the fp32 product rounded to IN_DT.
-template <int IN_DT, bool REQ, int SFMT>
+// IN_DT: the fp32 product, with ROUND rounded to IN_DT.
+template <int IN_DT, bool REQ, int SFMT, bool ROUND>
 __device__ __forceinline__ void rw_load8(const void *x, int64_t idx, float srow, float (&v)[8]) {
     if constexpr (!REQ) {
         load8<IN_DT>(x, idx, v);
@@ -521,16 +535,19 @@ __device__ __forceinline__ void rw_load8(const void *x, int64_t idx, float srow,
             }
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < 8; j += 2) {
             v[j] *= srow;
-            if constexpr (IN_DT == PTA_BF16) v[j] = bf16_bits_to_f32(f32_to_bf16_bits(v[j]));
-            if constexpr (IN_DT == PTA_F16) v[j] = f16_bits_to_f32(f32_to_f16_bits(v[j]));
+            v[j + 1] *= srow;
+            if constexpr (ROUND) round16<IN_DT>(v[j], v[j + 1]);
         }
     }
 }
 
 // Partial column amax, vector form: 512 columns x RW_CH rows per workgroup, 16
-// bytes (8 columns) per lane, the rows split over the 4 waves.
+// bytes (8 columns) per lane, the rows split over the 4 waves.  Rounding keeps the
+// order, so fp8 sources round the maximum of the products instead of each product:
+// with 4 VALU operations per element where there were 15, memory bounds it (MI355X,
+// 14336 x 4096: 26 -> 10.8 us; 8192 x 4096: 17 -> 7.9).
 template <int IN_DT, bool REQ, int SFMT>
 __global__ __launch_bounds__(NT) void rw_colv_partial_kernel(const void *x, const float *srow, int64_t len,
                                                               int64_t inner, float *partial, int64_t nchunk) {
@@ -544,19 +561,26 @@ __global__ __launch_bounds__(NT) void rw_colv_partial_kernel(const void *x, cons
 #pragma unroll 8
         for (int64_t r = r0 + wave; r < r1; r += 4) {
             float v[8];
-            rw_load8<IN_DT, REQ, SFMT>(x, (o * len + r) * inner + n, REQ ? srow[r] : 0.0f, v);
+            rw_load8<IN_DT, REQ, SFMT, false>(x, (o * len + r) * inner + n, REQ ? srow[r] : 0.0f, v);
+            // a product is never a signalling NaN
 #pragma unroll
-            for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], absq(v[j]));
+            for (int j = 0; j < 8; ++j) m[j] = fmaxf(m[j], REQ ? fabsf(v[j]) : absq(v[j]));
         }
     }
     *reinterpret_cast<float4 *>(&s[wave][lane * 8])     = make_float4(m[0], m[1], m[2], m[3]);
     *reinterpret_cast<float4 *>(&s[wave][lane * 8 + 4]) = make_float4(m[4], m[5], m[6], m[7]);
     __syncthreads();
+    float a[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int k = threadIdx.x + NT * h;
-        if (n0 + k < inner)
-            partial[(o * nchunk + c) * inner + n0 + k] = amax2(amax2(s[0][k], s[1][k]), amax2(s[2][k], s[3][k]));
+        a[h] = amax2(amax2(s[0][k], s[1][k]), amax2(s[2][k], s[3][k]));
+    }
+    if constexpr (REQ) round16<IN_DT>(a[0], a[1]);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = threadIdx.x + NT * h;
+        if (n0 + k < inner) partial[(o * nchunk + c) * inner + n0 + k] = a[h];
     }
 }
 
@@ -566,8 +590,9 @@ __global__ __launch_bounds__(NT) void rw_colv_partial_kernel(const void *x, cons
 // tile passes through LDS as in byte_transpose.h.  Bound by memory; MI355X,
 // 8192 x 14336 bf16: amax + finalize + transposed quantize 43.5 + 5.4 + 67 us
 // (124 + 33 + 149 us with one element per lane and load, plus 42 us for the byte
-// transpose).  Re-quantizing 14336 x 4096 fp8 rows: 26 + 5.5 + 30 us, where the
-// dequantized copy cost 28 + 42 + 55 + 49 us and the byte transpose 23 us.
+// transpose).  Re-quantizing 14336 x 4096 fp8 rows: 10.8 + 5.4 + 21.8 us, where the
+// dequantized copy cost 28 + 42 + 55 + 49 us and the byte transpose 23 us (the
+// quantize pass 31 us with the rounding to 16 bits in integer operations).
 template <int IN_DT, bool REQ, int SFMT, int FMT, bool TRANS>
 __global__ __launch_bounds__(NT) void rw_colv_quant_kernel(const void *x, const float *srow, int64_t len,
                                                             int64_t inner, const float *scale, uint8_t *q) {
@@ -588,8 +613,8 @@ __global__ __launch_bounds__(NT) void rw_colv_quant_kernel(const void *x, const 
         if (in && r < rows) {
             const int64_t idx = (o * len + m0 + r) * inner + n;
             const float   sr  = REQ ? srow[m0 + r] : 0.0f;
-            rw_load8<IN_DT, REQ, SFMT>(x, idx, sr, a);
-            rw_load8<IN_DT, REQ, SFMT>(x, idx + 8, sr, b);
+            rw_load8<IN_DT, REQ, SFMT, true>(x, idx, sr, a);
+            rw_load8<IN_DT, REQ, SFMT, true>(x, idx + 8, sr, b);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) { v[i][j] = a[j]; v[i][8 + j] = b[j]; }

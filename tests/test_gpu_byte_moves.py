@@ -112,3 +112,25 @@ def test_rowwise_columns_transposed(shape, fmt, dtype):
     q, s = quantize_fp8_rowwise_cols_t_impl(r, fmt, rs, dtype)
     wq, ws = want((r.float().cpu() * rs.cpu()).to(dtype))
     assert torch.equal(q.view(torch.uint8).cpu(), wq) and torch.equal(s.cpu(), ws)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt", [E4, torch.float8_e5m2])
+def test_rowwise_columns_of_special_rows(fmt, dtype):
+    """The column maximum is rounded once, after the maximum: every byte pattern,
+    products past the type's largest value and below its smallest, and row scales
+    that are zero, infinite or NaN give what quantizing the dequantized rows gives."""
+    from primus_turbo.pytorch.kernels.quantization.quantization_impl import quantize_fp8_rowwise_cols_t_impl
+
+    r = _bytes((208, 528), 5).view(fmt)
+    rs = torch.logspace(-42, 36, 208)
+    rs[3], rs[70], rs[131] = 0.0, float("inf"), float("nan")
+    keep = torch.arange(528) % 3 > 0  # a third of the columns has every special value
+    clean = torch.randn((208, 528), generator=torch.Generator().manual_seed(6)).to(fmt)
+    r = torch.where(keep[None], clean.view(torch.uint8), r.view(torch.uint8)).cuda().view(fmt)
+    for scales in (rs, torch.logspace(-9, 2, 208)):
+        sc = scales.cuda()[:, None].contiguous()
+        q, s = quantize_fp8_rowwise_cols_t_impl(r, fmt, sc, dtype)
+        wq, ws = quantize_fp8_rowwise_cols_t_impl((r.float() * sc).to(dtype), fmt)
+        assert torch.equal(s.view(torch.int32), ws.view(torch.int32))
+        assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8))
