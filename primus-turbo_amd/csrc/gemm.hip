@@ -68,16 +68,12 @@ int64_t split_tiles(int64_t tiles, int64_t K, int cus, int kind) {
     return cdiv(K, BK) * BK >= kmin ? tiles : 0;
 }
 
-// the same for any kind of scales (workspace sizes)
-int64_t split_tiles_most(int64_t tiles, int64_t K, int cus) {
-    int64_t n = 0;
-    for (int k = SPLIT_PLAIN; k <= SPLIT_1D_1D; ++k) n = n > split_tiles(tiles, K, cus, k) ? n : split_tiles(tiles, K, cus, k);
-    return n;
-}
-
-int split_kind(int sm, bool a2d, bool b2d) {
+// 1-D by 1-D scales are known by the extents of their arrays (one scale per row
+// and K block on both sides), which the size queries know too
+int split_kind(int sm, int64_t M, int64_t N, int64_t K, int64_t sa_bytes, int64_t sb_bytes) {
     if (sm == SM_TENSOR || sm == SM_ROW) return SPLIT_PLAIN;
-    return sm == SM_BLOCK && !a2d && !b2d ? SPLIT_1D_1D : SPLIT_SCALED;
+    const int64_t kb4 = cdiv(K, BK) * 4;
+    return sm == SM_BLOCK && sa_bytes == M * kb4 && sb_bytes == N * kb4 ? SPLIT_1D_1D : SPLIT_SCALED;
 }
 
 constexpr int64_t SPLIT_TILE_BYTES = int64_t(BM) * BN * 4;
@@ -111,7 +107,9 @@ int gemm_nt_launch(const uint8_t *a, int fa, int64_t lda, const uint8_t *b, int 
     g.aligned_c = ((ldc * (out_dt == PTA_F32 ? 4 : 2)) % 16 == 0) && aligned16(c);
     if (split_ws != nullptr && !stream_capturing(st)) {
         // a graph would replay the call tag, so captured calls do not split
-        const int64_t ns = split_tiles(int64_t(g.tiles_m) * g.tiles_n, K, device_cu_count(), split_kind(sm, a2d, b2d));
+        int kind = split_kind(sm, M, N, K, sa_bytes, sb_bytes);
+        if ((a2d || b2d) && kind == SPLIT_1D_1D) kind = SPLIT_SCALED;
+        const int64_t ns = split_tiles(int64_t(g.tiles_m) * g.tiles_n, K, device_cu_count(), kind);
         if (ns > 0) {
             const uint64_t tag = next_call_tag();
             const WaitPlan w   = wait_plan(tag, SPLIT_SPIN_LIMIT);
@@ -267,7 +265,9 @@ extern "C" size_t pta_gemm_fp8_workspace_size(int64_t M, int64_t N, int64_t K, i
     size_t ws = 0;
     if (trans_a) ws += static_cast<size_t>(cdiv(M * K, 256) * 256);
     if (!trans_b) ws += static_cast<size_t>(cdiv(N * K, 256) * 256);
-    ws += static_cast<size_t>(split_ws_bytes(split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
+    const int sm   = gran_to_sm(granularity);
+    const int kind = sm == SM_TENSOR || sm == SM_ROW ? SPLIT_PLAIN : sm == SM_BLOCK && trans_a ? SPLIT_1D_1D : SPLIT_SCALED;
+    ws += static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), kind)));
     return ws;
 }
 
@@ -320,8 +320,8 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
         wsp += cdiv(N * K, 256) * 256;
     }
     // what remains of the workspace holds the K split's partial tiles
-    uint8_t      *split_ws  = split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count()) > 0 ? wsp : nullptr;
     const int64_t split_off = workspace != nullptr ? wsp - static_cast<uint8_t *>(workspace) : 0;
+    uint8_t      *split_ws  = static_cast<size_t>(split_off) < need ? wsp : nullptr;
     // scale strides in the NT view
     bool    a2d = false, b2d = false;
     int64_t sa_m = 0, sa_k = 0, sb_m = 0, sb_k = 0;
@@ -369,7 +369,8 @@ static bool strided_small_path(int64_t M, int64_t N, int64_t K, int64_t lda, int
 static size_t strided_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t sa_bytes,
                                int64_t sb_bytes, int sm) {
     if (strided_small_path(M, N, K, lda, ldb, sa_bytes, sb_bytes, sm)) return 0;
-    return static_cast<size_t>(split_ws_bytes(split_tiles_most(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
+    const int kind = split_kind(sm, M, N, K, sa_bytes, sb_bytes);
+    return static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), kind)));
 }
 
 // choose: pick the small-tile kernel or the K split as pta_gemm_fp8 does

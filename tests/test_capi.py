@@ -97,6 +97,23 @@ def test_strided_entry_workspace_queries():
     assert q(0, 1024, 1024, 1, 1024, 1024, 4, 4) == 0
 
 
+def test_split_workspace_of_1d_by_1d_scales():
+    """Blockwise with one scale per row and K block on both sides splits from 16 K
+    blocks; the strided query knows it by the scales' extents, the other by the layout."""
+    from primus_turbo.pytorch import _C
+
+    q = lambda M, N, K, a, b: _C.query("pta_gemm_fp8_nt_strided_ws_size", M, N, K, 3, K, K, a, b)  # noqa: E731
+    split = 256 * 256 * 4
+    assert q(2048, 2048, 2048, 2048 * 16 * 4, 2048 * 16 * 4) >= 64 * split
+    assert q(2048, 2048, 2048, 2048 * 16 * 4, 16 * 16 * 4) == 0      # 128 x 128 scales on one side
+    assert q(2048, 2048, 1920, 2048 * 15 * 4, 2048 * 15 * 4) == 0    # 15 K blocks
+    assert q(2304, 3072, 2048, 2304 * 16 * 4, 3072 * 16 * 4) == 0    # past 96 tiles
+    ws = lambda ta, tb: _C.query("pta_gemm_fp8_workspace_size", 2056, 4096, 2048, ta, tb, 3)  # noqa: E731
+    assert ws(0, 1) == 0                                             # 144 tiles
+    ws = lambda ta, tb: _C.query("pta_gemm_fp8_workspace_size", 2044, 2560, 2048, ta, tb, 3)  # noqa: E731
+    assert ws(0, 1) == 0 and ws(1, 0) >= 80 * split + (2044 + 2560) * 2048
+
+
 def test_argument_errors_of_the_grouped_and_moe_entries():
     """Host-side argument checks of the newer entry points fire before any HIP
     call, with a message naming the problem (so no GPU is needed)."""
