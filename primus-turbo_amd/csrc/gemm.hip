@@ -68,6 +68,12 @@ int64_t split_tiles(int64_t tiles, int64_t K, int cus, int kind) {
     return cdiv(K, BK) * BK >= kmin ? tiles : 0;
 }
 
+// Tiles whose split a call insists on having a workspace for; the cut and the 1-D
+// by 1-D problems that split beyond these run whole where it is missing.
+int64_t split_tiles_required(int64_t tiles, int64_t K, int cus) {
+    return K % BK == 0 ? split_tiles(tiles, K, cus, SPLIT_PLAIN) : 0;
+}
+
 // 1-D by 1-D scales are known by the extents of their arrays (one scale per row
 // and K block on both sides), which the size queries know too
 int split_kind(int sm, int64_t M, int64_t N, int64_t K, int64_t sa_bytes, int64_t sb_bytes) {
@@ -298,10 +304,17 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
         PTA_CHECK_LAUNCH();
         return PTA_OK;
     }
-    const size_t need = pta_gemm_fp8_workspace_size(M, N, K, trans_a, trans_b, granularity);
+    const bool   small = small_path(M, N, K, trans_a, trans_b, sm);
+    const size_t want  = pta_gemm_fp8_workspace_size(M, N, K, trans_a, trans_b, granularity);
+    size_t       need  = 0;
+    if (!small) {
+        if (trans_a) need += static_cast<size_t>(cdiv(M * K, 256) * 256);
+        if (!trans_b) need += static_cast<size_t>(cdiv(N * K, 256) * 256);
+        need += static_cast<size_t>(split_ws_bytes(split_tiles_required(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
+    }
     PTA_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                   "workspace of %zu bytes required", need);
-    if (small_path(M, N, K, trans_a, trans_b, sm))
+    if (small)
         return gemm_small_nt(a, a_fmt, a_scale, trans_a, b, b_fmt, b_scale, trans_b, c, c_dtype, trans_c, M, N, K,
                              sm, st);
 
@@ -321,7 +334,7 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
     }
     // what remains of the workspace holds the K split's partial tiles
     const int64_t split_off = workspace != nullptr ? wsp - static_cast<uint8_t *>(workspace) : 0;
-    uint8_t      *split_ws  = static_cast<size_t>(split_off) < need ? wsp : nullptr;
+    uint8_t      *split_ws  = workspace != nullptr && static_cast<size_t>(split_off) < want && workspace_bytes >= want ? wsp : nullptr;
     // scale strides in the NT view
     bool    a2d = false, b2d = false;
     int64_t sa_m = 0, sa_k = 0, sb_m = 0, sb_k = 0;
@@ -408,7 +421,9 @@ static int nt_strided(const void *a, int a_fmt, int64_t lda, const void *b, int 
     hipStream_t st       = as_stream(stream);
     uint8_t    *split_ws = nullptr;
     if (choose) {
-        const size_t need = strided_ws_bytes(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm);
+        const size_t want = strided_ws_bytes(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm);
+        const size_t need = want == 0 ? 0 : static_cast<size_t>(split_ws_bytes(
+                                                split_tiles_required(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
         PTA_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                       "workspace of %zu bytes required", need);
         if (strided_small_path(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm)) {
@@ -424,7 +439,7 @@ static int nt_strided(const void *a, int a_fmt, int64_t lda, const void *b, int 
             }
             return small_dispatch(g, false, false, a_fmt, b_fmt, c_dtype, sm, st);
         }
-        if (need > 0) split_ws = static_cast<uint8_t *>(workspace);
+        if (want > 0 && workspace != nullptr && workspace_bytes >= want) split_ws = static_cast<uint8_t *>(workspace);
     }
     return gemm_nt_launch(static_cast<const uint8_t *>(a), a_fmt, lda, static_cast<const uint8_t *>(b), b_fmt,
                           ldb, c, c_dtype, ldc, M, N, K, sm, a_scale_2d != 0, b_scale_2d != 0, a_scale, sa_m,

@@ -112,3 +112,22 @@ def test_padded_quantized_rows(shape, dtype):
         q, s, qt = quant_fp8_blockwise_for_weight_impl(x.cuda(), torch.float8_e4m3fn, 128, with_transpose=True, pad16=pad)
         assert np.array_equal(u8(q)[:, :N], wq) and not u8(q)[:, N:].any() and np.array_equal(s.cpu().numpy(), ws)
         assert np.array_equal(u8(qt)[:, :M], wq.T) and not u8(qt)[:, M:].any()
+
+
+@pytest.mark.parametrize("K", [2048, 4016])
+def test_split_without_its_workspace_runs_whole(K):
+    """A problem that splits only for its 1-D by 1-D scales or with a cut K takes a
+    call without the partial tiles' workspace, bit for bit the unsplit kernel."""
+    from primus_turbo.pytorch import _C
+    from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_nt
+
+    M, N = 1024, 4096
+    qa, qb, g, nt = _strided_args(M, N, K, "BLOCK_1Dx1D", 70)
+    ref = gemm_fp8_nt(qa, qb, torch.bfloat16, g, **nt, large_tiles_only=True)
+    real = _C.workspace
+    try:
+        _C.workspace = lambda n, device: None
+        got = gemm_fp8_nt(qa, qb, torch.bfloat16, g, **nt)
+    finally:
+        _C.workspace = real
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
