@@ -97,6 +97,8 @@ def quantize_fp8_rowwise_cols_t_impl(
     dequantization to ``src_dtype`` would be."""
     M, N = x.shape
     x = x.contiguous()
+    if x.data_ptr() % 16:  # a view at an odd offset: the kernel has 16-byte loads only
+        x = x.clone()
     q_t = torch.empty((N, M), dtype=out_dtype, device=x.device)
     scale_inv = torch.empty((N,), dtype=torch.float32, device=x.device)
     ws = _C.workspace(_C.query("pta_quantize_fp8_rowwise_workspace_size", 1, M, N), x.device)

@@ -134,3 +134,22 @@ def test_rowwise_columns_of_special_rows(fmt, dtype):
         wq, ws = quantize_fp8_rowwise_cols_t_impl((r.float() * sc).to(dtype), fmt)
         assert torch.equal(s.view(torch.int32), ws.view(torch.int32))
         assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8))
+
+
+@pytest.mark.parametrize("trans_b", [True, False])
+def test_rowwise_layer_takes_a_gradient_at_an_odd_offset(trans_b):
+    """A contiguous gradient whose storage starts off a 16-byte boundary gives the
+    bits that an aligned copy of it gives."""
+    from primus_turbo.pytorch.core.low_precision import Float8QuantConfig
+    from primus_turbo.pytorch.ops import gemm_fp8
+
+    M, N, K = 144, 272, 128
+    g = torch.Generator().manual_seed(9)
+    a = torch.randn((M, K), generator=g).bfloat16().cuda().requires_grad_()
+    b = torch.randn((N, K) if trans_b else (K, N), generator=g).bfloat16().cuda().requires_grad_()
+    config = Float8QuantConfig(granularity=ScalingGranularity.ROWWISE)
+    grad = torch.randn(M * N + 1, generator=g).bfloat16().cuda()[1:].view(M, N)
+    assert grad.data_ptr() % 16
+    got = torch.autograd.grad(gemm_fp8(a, b, trans_b=trans_b, config=config), (a, b), grad)
+    want = torch.autograd.grad(gemm_fp8(a, b, trans_b=trans_b, config=config), (a, b), grad.clone())
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
