@@ -80,6 +80,14 @@ int pta_last_wait_status(uint64_t *tag, int64_t *status_offset);
  * path only. */
 void pta_test_force_wait_giveup(int on);
 
+/* Test hook: the reads that the GEMM kernels' loads of one operand [rows, K] (row
+ * stride ld) and its blockwise / MX scales (scale_elem_bytes 4 or 1, 0: none; strides
+ * and extent as in pta_gemm_fp8_nt_strided) could make outside them, under any of
+ * the ways in which a buffer load's range check may treat the scalar offset.  Host
+ * only; -1 for a bad shape. */
+int64_t pta_test_gemm_stray_reads(int64_t rows, int64_t K, int64_t ld, int scale_elem_bytes, int scale_2d,
+                                  int64_t s_m, int64_t s_k, int64_t s_bytes);
+
 /* ============================================================================
  * Quantization
  * ========================================================================== */

@@ -24,6 +24,7 @@
 // (4 FMAs per MFMA) overlaps the matrix pipe.
 #pragma once
 #include "common.h"
+#include "gemm_addr.h"
 
 namespace pta {
 namespace gemm_detail {
@@ -31,8 +32,6 @@ namespace gemm_detail {
 typedef int   v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 256, BK = 128;
-constexpr int BN = 256;                     // default tile width (128 for tail tiles)
 constexpr int WGM = 4, WGN = 2;             // wave grid
 constexpr int NWAVES = WGM * WGN;
 constexpr int NTHR = 64 * NWAVES;
@@ -144,8 +143,7 @@ __device__ __forceinline__ void store4(void *c, int64_t idx, float x0, float x1,
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, int64_t bytes) {
-    const int32_t n = bytes > 0x7fffffff ? 0x7fffffff : static_cast<int32_t>(bytes);
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), static_cast<short>(0), n, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), static_cast<short>(0), desc_records(bytes), 0x00020000);
 }
 __device__ __forceinline__ uint4 bload16(rsrc_t r, int voff, int soff) {
     return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
@@ -171,10 +169,9 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 // buffer descriptor as an SGPR quad for inline asm (wave-uniform inputs)
 __device__ __forceinline__ v4i make_desc(const void *p, int64_t bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(p);
-    const int32_t  n = bytes > 0x7fffffff ? 0x7fffffff : static_cast<int32_t>(bytes);
     return v4i{__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(a))),
                __builtin_amdgcn_readfirstlane(static_cast<int>((a >> 32) & 0xffff)),
-               __builtin_amdgcn_readfirstlane(n), 0x00020000};
+               __builtin_amdgcn_readfirstlane(desc_records(bytes)), 0x00020000};
 }
 
 // LDS-DMA: N bytes per lane from desc[voff + soff] into LDS at m0 + N * lane.  The
@@ -421,62 +418,60 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     // of the B tile (b0, b1).  Each wave moves 16 rows of every item, 8 rows per
     // instruction; lane i fills LDS chunk i of that 1 KB span = row i/8,
     // physical chunk i%8, which holds logical chunk (i%8) ^ swz(row).
-    const int rowsA = static_cast<int>(min<int64_t>(M - m0, BM)), rowsB = static_cast<int>(min<int64_t>(N - n0, BN_));
-    v4i       dA[2], dB[2];
+    v4i dA[2], dB[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int ra = rowsA - 128 * h, rb = rowsB - 128 * h;
-        dA[h] = make_desc(A + (m0 + 128 * h) * g.lda, ra > 0 ? (min(ra, 128) - 1) * g.lda + K : 0);
-        dB[h] = make_desc(B + (n0 + 128 * h) * g.ldb, rb > 0 ? (min(rb, 128) - 1) * g.ldb + K : 0);
+        dA[h] = make_desc(A + (m0 + half_start(M - m0, h)) * g.lda, half_bytes(half_rows(M - m0, h), g.lda, K));
+        dB[h] = make_desc(B + (n0 + half_start(N - n0, h)) * g.ldb, half_bytes(half_rows(N - n0, h), g.ldb, K));
     }
     const int lr = lane >> 3, lp = lane & 7;
     const int ch = lp ^ lr;            // rows of one DMA are 8 apart: same swizzle
     int       vA[2], vB[2];
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
-        vA[d] = (wave * 16 + 8 * d + lr) * static_cast<int>(g.lda) + 16 * ch;
-        vB[d] = (wave * 16 + 8 * d + lr) * static_cast<int>(g.ldb) + 16 * ch;
+        vA[d] = lane_off(wave * 16 + 8 * d + lr, g.lda, ch);
+        vB[d] = lane_off(wave * 16 + 8 * d + lr, g.ldb, ch);
     }
     // chunks of the last K block that lie past K read out of range, as zeros
-    const int  ktail = (K % BK) != 0 ? nk - 1 : 0x7fffffff;
-    const bool koob  = (nk - 1) * BK + 16 * ch >= K;
+    const int  ktail = cut_block(nk, K);
+    const bool koob  = past_k(nk, K, ch);
     // per-K-block scales (blockwise fp32, MX four E8M0 bytes): one dword per A row
-    // (waves 0-3, 64 rows each) and per B row (waves 4-7) into a ring of four slots
+    // (waves 0-3, 64 rows each) and per B row (waves 4-7) into a ring of four slots;
+    // rows past the operand's last read its scales (nothing of them is stored)
     constexpr bool HAS_S = SM == SM_BLOCK || SM == SM_MX;
     v4i            dS{};
     int            vS = 0, ksS = 0;
     if constexpr (HAS_S) {
         constexpr int es = SM == SM_MX ? 1 : 4;
         const bool    isA = wave < 4;
-        const int64_t r   = (isA ? m0 : n0) + 64 * (wave & 3) + lane;
+        const int64_t r   = scale_row((isA ? m0 : n0) + 64 * (wave & 3) + lane, isA ? M : N);
         dS  = isA ? make_desc(g.sa, g.sa_bytes) : make_desc(SB, g.sb_bytes);
-        vS  = static_cast<int>(((isA ? A2D : B2D) ? (r >> 7) : r) * (isA ? g.sa_m : g.sb_m)) * es;
+        vS  = scale_off(r, isA ? A2D : B2D, isA ? g.sa_m : g.sb_m, es);
         ksS = static_cast<int>(isA ? g.sa_k : g.sb_k) * es;
     }
     // The part-th item of K block kb (part 0: a0 and the scales, 1: b0, 2: a1, 3:
     // b1); nothing past the last block: skipped by the ping-pong loop and the
     // persistent kernels, read out of range (a descriptor with no records; LDS gets
-    // zeros) by the other interleaved loops, which the skip makes 1-1.7% slower
-    // (MX 8192 x 28672 x 8192 1344 against 1367 us; grouped MX, persistent, 1020
-    // against 1004).
+    // zeros, and a scale slot that is not read again the last block's) by the other
+    // interleaved loops, which the skip makes 1-1.7% slower (MX 8192 x 28672 x 8192
+    // 1344 against 1367 us; grouped MX, persistent, 1020 against 1004).
     constexpr bool PINGPONG = SM == SM_TENSOR || SM == SM_ROW || (SM == SM_BLOCK && B2D);
     constexpr bool SKIP     = PINGPONG || PERSIST;
     auto           issue    = [&](int kb, int part) {
-        const int      k0 = kb * BK, h = part >> 1, ks = (kb + static_cast<int>(kb_base)) * ksS;
+        const int      h = part >> 1, last = SKIP ? kb + 1 : nk; // skipped blocks need no offsets
+        const int      k0 = item_soff(kb, last), ks = (scale_block(kb, last) + static_cast<int>(kb_base)) * ksS;
         const uint32_t ls = lds0 + SBASE_ + (kb & 3) * SSLOT_ + wave * 256;
-        const uint32_t l  = lds0 + (kb & 1) * STAGE_ + (part & 1) * TILE_A_BYTES + h * 128 * BK + wave * 16 * BK;
+        const uint32_t l  = lds0 + (kb & 1) * STAGE_ + (part & 1) * TILE_A_BYTES + h * HALF * BK + wave * 16 * BK;
         const bool     oob = kb >= ktail && koob;
-        const int      v0  = oob ? 0x7fffffff - 64 : ((part & 1) ? vB[0] : vA[0]);
-        const int      v1  = oob ? 0x7fffffff - 64 : ((part & 1) ? vB[1] : vA[1]);
+        const int      v0  = oob ? OOB_LANE : ((part & 1) ? vB[0] : vA[0]);
+        const int      v1  = oob ? OOB_LANE : ((part & 1) ? vB[1] : vA[1]);
         v4i            d   = (part & 1) ? dB[h] : dA[h];
         if constexpr (SKIP) {
             if (HAS_S && part == 0) dma4_if(kb, nk, ls, vS, dS, ks);
             dma16x2_if(kb, nk, l, v0, v1, d, k0);
         } else {
-            v4i ds = dS;
-            ds[2]  = kb < nk ? ds[2] : 0;
-            d[2]   = kb < nk ? d[2] : 0;
-            if (HAS_S && part == 0) dma4(ls, vS, ds, ks);
+            d[2] = item_records(d[2], kb, nk);
+            if (HAS_S && part == 0) dma4(ls, vS, dS, ks);
             dma16(l, v0, d, k0);
             dma16(l + 8 * BK, v1, d, k0);
         }
@@ -727,7 +722,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
             }
         }
     }
-    // DMAs past the last K block still write zeros to LDS
+    // DMAs past the last K block still write to LDS
     if constexpr (!SKIP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // ---- K split: the first half hands its accumulators to the second -------

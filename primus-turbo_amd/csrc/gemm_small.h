@@ -224,21 +224,21 @@ __global__ __launch_bounds__(SNTHR) void gemm_small_kernel(const SmallArgs g) {
     int          sa_vo[STM], sb_vo[STN][4];
 #pragma unroll
     for (int i = 0; i < STM; ++i) {
-        const int64_t m = min<int64_t>(m0 + wm * WTM + 16 * i + fr, M - 1);
-        if constexpr (SM == SM_BLOCK) sa_vo[i] = static_cast<int>((g.a2d ? (m >> 7) : m) * g.sa_m) * 4;
-        else if constexpr (SM == SM_MX) sa_vo[i] = static_cast<int>(m * g.sa_m) + fg;
+        const int64_t m = gemm_detail::scale_row(m0 + wm * WTM + 16 * i + fr, M);
+        if constexpr (SM == SM_BLOCK) sa_vo[i] = gemm_detail::scale_off(m, g.a2d, g.sa_m, 4);
+        else if constexpr (SM == SM_MX) sa_vo[i] = gemm_detail::scale_off(m, false, g.sa_m, 1) + fg;
     }
 #pragma unroll
     for (int j = 0; j < STN; ++j) {
         if constexpr (SM == SM_BLOCK) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t nc = min<int64_t>(n0 + wn * WTN + 16 * j + 4 * fg + r, N - 1);
-                sb_vo[j][r] = static_cast<int>((g.b2d ? (nc >> 7) : nc) * g.sb_m) * 4;
+                const int64_t nc = gemm_detail::scale_row(n0 + wn * WTN + 16 * j + 4 * fg + r, N);
+                sb_vo[j][r] = gemm_detail::scale_off(nc, g.b2d, g.sb_m, 4);
             }
         } else if constexpr (SM == SM_MX) {
-            const int64_t n = min<int64_t>(n0 + wn * WTN + 16 * j + fr, N - 1);
-            sb_vo[j][0] = static_cast<int>(n * g.sb_m) + fg;
+            const int64_t n = gemm_detail::scale_row(n0 + wn * WTN + 16 * j + fr, N);
+            sb_vo[j][0] = gemm_detail::scale_off(n, false, g.sb_m, 1) + fg;
         }
     }
 
@@ -246,8 +246,9 @@ __global__ __launch_bounds__(SNTHR) void gemm_small_kernel(const SmallArgs g) {
         const int k0 = kb * SBK;
         load_operand<AKM, SBM>(rA, lda, k0, Ki, s.a);
         load_operand<BKM, SBN>(rB, ldb, k0, Ki, s.b);
+        const int kbs = gemm_detail::scale_block(kb, nk); // scales past K: read again, never used
         if constexpr (SM == SM_BLOCK) {
-            const int ka = static_cast<int>(kb * g.sa_k) * 4, kbb = static_cast<int>(kb * g.sb_k) * 4;
+            const int ka = static_cast<int>(kbs * g.sa_k) * 4, kbb = static_cast<int>(kbs * g.sb_k) * 4;
 #pragma unroll
             for (int i = 0; i < STM; ++i) s.sa[i] = gemm_detail::bload_f32(rSA, sa_vo[i], ka);
 #pragma unroll
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(SNTHR) void gemm_small_kernel(const SmallArgs g) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) s.sb[j][r] = gemm_detail::bload_f32(rSB, sb_vo[j][r], kbb);
         } else if constexpr (SM == SM_MX) {
-            const int ka = static_cast<int>(kb * g.sa_k), kbb = static_cast<int>(kb * g.sb_k);
+            const int ka = static_cast<int>(kbs * g.sa_k), kbb = static_cast<int>(kbs * g.sb_k);
 #pragma unroll
             for (int i = 0; i < STM; ++i) s.ea[i] = gemm_detail::bload_u8(rSA, sa_vo[i], ka);
 #pragma unroll

@@ -1,7 +1,9 @@
-"""The 256 x 256 GEMM's LDS-DMAs, checked without a GPU."""
+"""The loads of the GEMM kernels, checked without a GPU."""
 
 import os
 import re
+
+import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "primus-turbo_amd", "csrc")
 
@@ -27,3 +29,24 @@ def test_m0_is_written_an_instruction_ahead_of_the_dma_that_reads_it():
                 assert any(p.startswith("s_mov_b32 m0") for p in block[:i]), (name, block)
                 assert not block[i - 1].startswith("s_mov_b32 m0"), (name, block)
     assert dmas >= 4
+
+
+@pytest.mark.parametrize("rows", [1, 16, 127, 128, 129, 255, 256, 257, 384, 385, 700])
+@pytest.mark.parametrize("K", [16, 112, 128, 144, 256, 400, 1152])
+@pytest.mark.parametrize("wider", [0, 48])
+def test_loads_stay_inside_the_operands(rows, K, wider):
+    """Partial tiles, half tiles without rows, a cut last K block, and the blocks past
+    it: no lane reads outside the operand or its scales, however the range check of a
+    buffer load treats the scalar offset."""
+    from primus_turbo.pytorch import _C
+
+    kb, ld = -(-K // 128), K + wider
+    stray = _C.load().pta_test_gemm_stray_reads
+    assert stray(rows, K, ld, 0, 0, 0, 0, 0) == 0
+    assert stray(rows, K, ld, 4, 0, kb, 1, rows * kb * 4) == 0            # [rows, K / 128]
+    assert stray(rows, K, ld, 4, 0, 1, rows, rows * kb * 4) == 0          # [K / 128, rows]
+    tiles = -(-rows // 128)
+    assert stray(rows, K, ld, 4, 1, kb, 1, tiles * kb * 4) == 0           # 128 x 128
+    assert stray(rows, K, ld, 4, 1, 1, tiles, tiles * kb * 4) == 0
+    assert stray(rows, K, ld, 1, 0, kb * 4, 4, rows * kb * 4) == 0        # E8M0, row-major
+    assert stray(rows, K, ld, 1, 0, 4, rows * 4, rows * kb * 4) == 0      # E8M0, K-major
