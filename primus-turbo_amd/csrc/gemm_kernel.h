@@ -177,17 +177,18 @@ __device__ __forceinline__ v4i make_desc(const void *p, int64_t bytes) {
 // LDS-DMA: N bytes per lane from desc[voff + soff] into LDS at m0 + N * lane.  The
 // instructions are hidden from the compiler's wait-count tracking on purpose:
 // completion is awaited explicitly (wait_dma_and_barrier).  The compiler's hazard
-// handling doesn't look inside either: a scalar write of M0 needs one instruction
-// between it and the DMA that reads it.
+// handling doesn't look inside either: a scalar write of M0 needs one wait state
+// before the DMA that reads it, and an SGPR that a VALU instruction wrote (a spilled
+// one read back by v_readlane) needs five.
 __device__ __forceinline__ void dma16(uint32_t lds_addr, int voff, v4i desc, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(desc),
                    "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(uint32_t lds_addr, int voff, v4i desc, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds"
                  :
                  : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(desc),
                    "s"(__builtin_amdgcn_readfirstlane(soff))
@@ -199,7 +200,7 @@ __device__ __forceinline__ void dma4(uint32_t lds_addr, int voff, v4i desc, int 
 // scheduling region, and the register allocator then spills 150-200 VGPRs.
 __device__ __forceinline__ void dma16x2_if(int kb, int nk, uint32_t lds_addr, int voff0, int voff1, v4i desc, int soff) {
     const uint32_t l = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile("s_mov_b32 m0, %1\n\ts_cmp_lt_i32 %0, %7\n\ts_cbranch_scc0 .Ldma%=\n\t"
+    asm volatile("s_mov_b32 m0, %1\n\ts_cmp_lt_i32 %0, %7\n\ts_cbranch_scc0 .Ldma%=\n\ts_nop 1\n\t"
                  "buffer_load_dwordx4 %3, %5, %6 offen lds\n\t"
                  "s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds\n.Ldma%=:"
                  :
@@ -208,7 +209,7 @@ __device__ __forceinline__ void dma16x2_if(int kb, int nk, uint32_t lds_addr, in
                  : "memory", "m0", "scc");
 }
 __device__ __forceinline__ void dma4_if(int kb, int nk, uint32_t lds_addr, int voff, v4i desc, int soff) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_cmp_lt_i32 %0, %5\n\ts_cbranch_scc0 .Ldma%=\n\t"
+    asm volatile("s_mov_b32 m0, %1\n\ts_cmp_lt_i32 %0, %5\n\ts_cbranch_scc0 .Ldma%=\n\ts_nop 1\n\t"
                  "buffer_load_dword %2, %3, %4 offen lds\n.Ldma%=:"
                  :
                  : "s"(kb), "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(desc),

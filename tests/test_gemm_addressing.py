@@ -50,3 +50,21 @@ def test_loads_stay_inside_the_operands(rows, K, wider):
     assert stray(rows, K, ld, 4, 1, 1, tiles, tiles * kb * 4) == 0
     assert stray(rows, K, ld, 1, 0, kb * 4, 4, rows * kb * 4) == 0        # E8M0, row-major
     assert stray(rows, K, ld, 1, 0, 4, rows * 4, rows * kb * 4) == 0      # E8M0, K-major
+
+
+def _wait_states(block):
+    """Wait states that a run of instructions gives (s_nop N: N + 1)."""
+    return sum(int(i.split()[1]) + 1 if i.startswith("s_nop") else 1 for i in block if not i.endswith(":"))
+
+
+def test_sgprs_written_by_the_vector_unit_are_ready_for_the_dma():
+    """A spilled SGPR comes back by v_readlane, which the compiler may put right ahead
+    of an asm statement: a buffer load that reads it needs five wait states."""
+    dmas = 0
+    for name in sorted(os.listdir(CSRC)):
+        for block in _asm_blocks(open(os.path.join(CSRC, name)).read()):
+            first = next((i for i, ins in enumerate(block) if ins.startswith("buffer_load")), None)
+            if first is not None:
+                dmas += 1
+                assert _wait_states(block[:first]) >= 5, (name, block)
+    assert dmas >= 4
