@@ -88,6 +88,12 @@ void pta_test_force_wait_giveup(int on);
 int64_t pta_test_gemm_stray_reads(int64_t rows, int64_t K, int64_t ld, int scale_elem_bytes, int scale_2d,
                                   int64_t s_m, int64_t s_k, int64_t s_bytes);
 
+/* Test hook: how pta_gemm_fp8_nt_strided_ws runs a problem with dense rows: 0 the
+ * small-tile kernel, 1 whole 256 x 256 tiles, 2 their K split (can_split: the call
+ * has the workspace); -1 for bad arguments. */
+int pta_test_gemm_route(int64_t M, int64_t N, int64_t K, int granularity, int64_t a_scale_bytes,
+                        int64_t b_scale_bytes, int can_split);
+
 /* ============================================================================
  * Quantization
  * ========================================================================== */
@@ -332,7 +338,7 @@ int pta_grouped_compute_padded_offs(const int64_t *offs, int64_t *padded_offs, i
  * (a quarter round: 24; 3/8 of a round with 1-D scales on both sides: 16), the
  * fp32 partial tiles of the K split (each tile then runs as two half-K workgroups;
  * not under stream capture).  Where K % 128 != 0 or fewer K blocks split only for
- * their scales, a call without that part runs whole.  Replaces gemm_fp8_impl
+ * their scales, a call without that part runs unsplit.  Replaces gemm_fp8_impl
  * (primus_turbo/pytorch/kernels/gemm/gemm_fp8_impl.py:438-467) and the native
  * hipblaslt/ck/turbo_gemm_fp8 ops behind it. */
 size_t pta_gemm_fp8_workspace_size(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b,

@@ -82,6 +82,12 @@ int split_kind(int sm, int64_t M, int64_t N, int64_t K, int64_t sa_bytes, int64_
     return sm == SM_BLOCK && sa_bytes == M * kb4 && sb_bytes == N * kb4 ? SPLIT_1D_1D : SPLIT_SCALED;
 }
 
+// the same by the operands' layout: both 1-D in the TN product only
+int layout_split_kind(int sm, int trans_a) {
+    if (sm == SM_TENSOR || sm == SM_ROW) return SPLIT_PLAIN;
+    return sm == SM_BLOCK && trans_a ? SPLIT_1D_1D : SPLIT_SCALED;
+}
+
 constexpr int64_t SPLIT_TILE_BYTES = int64_t(BM) * BN * 4;
 
 // byte offset of the status word in a K-split workspace for `n` split tiles
@@ -247,17 +253,35 @@ static bool block_on_128_tiles(int64_t M, int64_t N, int sm) {
     return sm == SM_BLOCK && cdiv(M, 128) * cdiv(N, 128) >= PTA_SMALL_T128_MIN;
 }
 
+// Whether K-contiguous operands of few enough tiles for the small-tile kernel run on
+// the 256 x 256 kernel all the same: from 48 tiles and 32 K blocks on, where the K
+// split runs (can_split: its workspace is there; a capturing stream, which doesn't
+// split either, keeps the large tiles, whole).
+// Measured (us; split, whole, small-tile kernel):
+//   tensorwise  1024x3328x4000 31.9 39.1 37.0   1024x4096x4000 31.6 39.5 32.6   1792x2560x4000 33.3 40.5 47.9
+//   blockwise   1024x3328x4000 35.0 44.3 51.4    768x4096x4000 34.6 45.1 38.7
+//   1-D by 1-D  1024x3328x4000 43.4 60.1 52.9    768x4096x8080 70.7 115.6 76.8
+//   MX          1024x4096x4096 33.0 40.5 41.8
+// At 48 tiles a cut K of 32 blocks doesn't pay for the split but for blockwise scales
+// (768x4096x4000 tensorwise 31.3 40.0 30.3, 1-D by 1-D 43.3 60.6 40.0).  Without the
+// split the small-tile kernel is the faster one, except for blockwise scales with
+// 128 x 128 blocks on one side past 48 tiles.
+static bool large_tiles_for(int64_t tiles, int64_t K, int sm, int kind, bool can_split) {
+    const int64_t kb = cdiv(K, BK);
+    if (tiles < 48 || kb < 32) return false;
+    const bool pays = K % BK == 0 || kind == SPLIT_SCALED || tiles > 48 || kb >= 36;
+    if (can_split && pays && split_tiles(tiles, K, device_cu_count(), kind) > 0) return true;
+    return sm == SM_BLOCK && kind == SPLIT_SCALED && tiles > 48;
+}
+
 // Whether pta_gemm_fp8 takes the small-tile kernel: few large tiles, K-major
 // operands with a row stride that is a multiple of 8 (8-byte K-row loads), and
 // every operand offset of the kernel within 32 bits.
-static bool small_path(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int sm) {
+static bool small_path(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int sm, bool can_split) {
     const bool    kmajor = trans_a || !trans_b;
     const int64_t tiles  = cdiv(M, BM) * cdiv(N, BN);
     if (tiles >= (kmajor ? PTA_SMALL_MAX_TILES_KMAJOR : PTA_SMALL_MAX_TILES)) return false;
-    // K-contiguous operands, a quarter of a round of 256 x 256 tiles or more
-    // and a long K: the large tiles with the K split are faster (blockwise
-    // 1024x4096x4096: 62 -> 45 us; at K = 2048 or with fewer tiles they are not)
-    if (!kmajor && tiles >= 48 && cdiv(K, 128) >= 32) return false;
+    if (!kmajor && large_tiles_for(tiles, K, sm, layout_split_kind(sm, trans_a), can_split)) return false;
     if (!kmajor && block_on_128_tiles(M, N, sm)) return false;
     const int64_t lim = int64_t(1) << 30;
     if (trans_a ? (M % 8 != 0 || (K + 1024) * M >= lim) : 64 * K >= lim) return false;
@@ -267,13 +291,13 @@ static bool small_path(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b
 
 extern "C" size_t pta_gemm_fp8_workspace_size(int64_t M, int64_t N, int64_t K, int trans_a,
                                               int trans_b, int granularity) {
-    if (small_path(M, N, K, trans_a, trans_b, gran_to_sm(granularity))) return 0;
+    const int sm = gran_to_sm(granularity);
+    if (small_path(M, N, K, trans_a, trans_b, sm, true)) return 0;
     size_t ws = 0;
     if (trans_a) ws += static_cast<size_t>(cdiv(M * K, 256) * 256);
     if (!trans_b) ws += static_cast<size_t>(cdiv(N * K, 256) * 256);
-    const int sm   = gran_to_sm(granularity);
-    const int kind = sm == SM_TENSOR || sm == SM_ROW ? SPLIT_PLAIN : sm == SM_BLOCK && trans_a ? SPLIT_1D_1D : SPLIT_SCALED;
-    ws += static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), kind)));
+    ws += static_cast<size_t>(split_ws_bytes(
+        split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), layout_split_kind(sm, trans_a))));
     return ws;
 }
 
@@ -304,7 +328,7 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
         PTA_CHECK_LAUNCH();
         return PTA_OK;
     }
-    const bool   small = small_path(M, N, K, trans_a, trans_b, sm);
+    bool         small = small_path(M, N, K, trans_a, trans_b, sm, true);
     const size_t want  = pta_gemm_fp8_workspace_size(M, N, K, trans_a, trans_b, granularity);
     size_t       need  = 0;
     if (!small) {
@@ -314,6 +338,9 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
     }
     PTA_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                   "workspace of %zu bytes required", need);
+    // large tiles chosen for a split that this call has no workspace for
+    if (!small && small_path(M, N, K, trans_a, trans_b, sm, false))
+        small = workspace == nullptr || workspace_bytes < want;
     if (small)
         return gemm_small_nt(a, a_fmt, a_scale, trans_a, b, b_fmt, b_scale, trans_b, c, c_dtype, trans_c, M, N, K,
                              sm, st);
@@ -370,10 +397,10 @@ extern "C" int pta_gemm_fp8(const void *a, int a_fmt, const void *a_scale, int t
 // NT rule of small_path, with the operands' row strides (and the scale
 // extents) in 32-bit reach of the small kernel's buffer offsets.
 static bool strided_small_path(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t sa_bytes,
-                               int64_t sb_bytes, int sm) {
+                               int64_t sb_bytes, int sm, bool can_split) {
     const int64_t tiles = cdiv(M, BM) * cdiv(N, BN);
     if (tiles >= PTA_SMALL_MAX_TILES) return false;
-    if (tiles >= 48 && cdiv(K, 128) >= 32) return false; // the K split is faster there
+    if (large_tiles_for(tiles, K, sm, split_kind(sm, M, N, K, sa_bytes, sb_bytes), can_split)) return false;
     if (block_on_128_tiles(M, N, sm)) return false;
     const int64_t lim = int64_t(1) << 30;
     return 64 * lda < lim && 64 * ldb < lim && sa_bytes < 2 * lim && sb_bytes < 2 * lim;
@@ -381,7 +408,7 @@ static bool strided_small_path(int64_t M, int64_t N, int64_t K, int64_t lda, int
 
 static size_t strided_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t sa_bytes,
                                int64_t sb_bytes, int sm) {
-    if (strided_small_path(M, N, K, lda, ldb, sa_bytes, sb_bytes, sm)) return 0;
+    if (strided_small_path(M, N, K, lda, ldb, sa_bytes, sb_bytes, sm, true)) return 0;
     const int kind = split_kind(sm, M, N, K, sa_bytes, sb_bytes);
     return static_cast<size_t>(split_ws_bytes(split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), kind)));
 }
@@ -426,7 +453,10 @@ static int nt_strided(const void *a, int a_fmt, int64_t lda, const void *b, int 
                                                 split_tiles_required(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count())));
         PTA_CHECK_ARG(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                       "workspace of %zu bytes required", need);
-        if (strided_small_path(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm)) {
+        bool small = strided_small_path(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm, true);
+        if (!small && strided_small_path(M, N, K, lda, ldb, a_scale_bytes, b_scale_bytes, sm, false))
+            small = workspace == nullptr || workspace_bytes < want;
+        if (small) {
             gemm_small::SmallArgs g{};
             g.a = static_cast<const uint8_t *>(a); g.b = static_cast<const uint8_t *>(b); g.c = c;
             g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldb = ldb; g.ldc = ldc;
@@ -474,4 +504,13 @@ extern "C" int pta_gemm_fp8_nt_strided_ws(const void *a, int a_fmt, int64_t lda,
     return nt_strided(a, a_fmt, lda, b, b_fmt, ldb, c, c_dtype, ldc, M, N, K, granularity, a_scale, sa_m, sa_k,
                       a_scale_2d, a_scale_bytes, b_scale, sb_m, sb_k, b_scale_2d, b_scale_bytes, true, workspace,
                       workspace_bytes, stream);
+}
+
+extern "C" int pta_test_gemm_route(int64_t M, int64_t N, int64_t K, int granularity, int64_t a_scale_bytes,
+                                   int64_t b_scale_bytes, int can_split) {
+    const int sm = gran_to_sm(granularity);
+    if (sm < 0 || M < 1 || N < 1 || K < 1) return -1;
+    if (strided_small_path(M, N, K, K, K, a_scale_bytes, b_scale_bytes, sm, can_split != 0)) return 0;
+    const int kind = split_kind(sm, M, N, K, a_scale_bytes, b_scale_bytes);
+    return can_split && split_tiles(cdiv(M, BM) * cdiv(N, BN), K, device_cu_count(), kind) > 0 ? 2 : 1;
 }

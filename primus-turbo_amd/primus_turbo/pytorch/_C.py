@@ -35,6 +35,7 @@ SIGNATURES = {
     "pta_last_wait_status": (_i32, [ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_int64)]),
     "pta_test_force_wait_giveup": (None, [_i32]),
     "pta_test_gemm_stray_reads": (_i64, [_i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64]),
+    "pta_test_gemm_route": (_i32, [_i64, _i64, _i64, _i32, _i64, _i64, _i32]),
     "pta_quantize_fp8_tensorwise_workspace_size": (_sz, [_i64]),
     "pta_quantize_fp8_tensorwise": (_i32, [_vp, _i32, _i64, _vp, _vp, _i32, _vp, _vp, _sz, _vp]),
     "pta_quantize_fp8_tensorwise_noalloc": (_i32, [_vp, _i32, _i64, _vp, _vp, _i32, _vp, _vp]),

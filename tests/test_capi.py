@@ -145,3 +145,31 @@ def test_wait_status_without_a_bounded_wait():
     assert lib.pta_last_wait_status(ctypes.byref(tag), ctypes.byref(off)) == 0
     assert off.value == -1
     assert lib.pta_last_wait_status(None, None) == -1
+
+
+def test_route_without_the_split():
+    """From 48 tiles and 32 K blocks on the 256 x 256 kernel runs for its K split: where
+    a call has no workspace for it the small-tile kernel, faster than whole 256 x 256
+    tiles, runs as it does below that line."""
+    from primus_turbo.pytorch import _C
+
+    SMALL, WHOLE, SPLIT = 0, 1, 2
+
+    def route(gran, M, N, K, both_1d=False):
+        kb = -(-K // 128) * 4
+        s = {1: (4, 4), 2: (M * 4, N * 4), 4: (M * kb, N * kb),
+             3: (M * kb, (N if both_1d else -(-N // 128)) * kb)}[gran]
+        return tuple(_C.load().pta_test_gemm_route(M, N, K, gran, *s, split) for split in (1, 0))
+
+    for gran in (1, 2):
+        assert route(gran, 1024, 4096, 4000) == (SPLIT, SMALL)
+        assert route(gran, 1024, 4096, 4096) == (SPLIT, SMALL)
+        assert route(gran, 768, 4096, 4000) == (SMALL, SMALL)   # 48 tiles, 32 K blocks, cut
+        assert route(gran, 768, 4096, 4640) == (SPLIT, SMALL)
+        assert route(gran, 768, 4096, 3840) == (SMALL, SMALL)   # 30 K blocks
+        assert route(gran, 4096, 4096, 4000) == (WHOLE, WHOLE)  # a whole round of tiles
+    assert route(3, 1024, 3328, 4000) == (SPLIT, WHOLE)         # 128 x 128 blocks on one side
+    assert route(3, 768, 4096, 4000) == (SPLIT, SMALL)
+    assert route(3, 1024, 3328, 4000, True) == (SPLIT, SMALL)
+    assert route(3, 768, 4096, 4000, True) == (SMALL, SMALL)
+    assert route(4, 768, 4096, 4096) == (SPLIT, SMALL)
