@@ -151,9 +151,6 @@ __device__ __forceinline__ uint4 bload16(rsrc_t r, int voff, int soff) {
 __device__ __forceinline__ float bload_f32(rsrc_t r, int voff, int soff) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
-__device__ __forceinline__ float4 bload_f32x4(rsrc_t r, int voff, int soff) {
-    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
 __device__ __forceinline__ int bload_u8(rsrc_t r, int voff, int soff) {
     return static_cast<int>(__builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0));
 }
@@ -501,9 +498,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     // and a half K blocks in flight (counted vmcnt waits, never a full drain) and
     // spread their issue over the step: 8 per wave and K block, addressed by SGPRs
     // and five VGPRs so that nothing spills.  Same K order and scaling
-    // order in both, so the same bits.  What bounds them now is power: the clock
-    // falls to 1.9-2.0 GHz, and a variant that issues no DMAs (wrong results) gains
-    // 16% of the time with 11% of the cycles.
+    // order in both, so the same bits.  What bounds them is idle matrix pipes first and
+    // the clock second.  Busy share and clock on one card, at 4096 x 18432 x 7168 (1-D
+    // by 1-D: 18432 x 7168 x 4096), and those of a loop of the same MFMAs and VALU
+    // instructions on registers alone:
+    //   tensorwise 77% at 1.69 GHz (99% at 2.01)     1x128 by 128x128 60% at 1.86 (98% at 1.78)
+    //   1x128 by 1x128 45% at 2.07 (72% at 1.97)     MX 65% at 1.89 (99% at 2.05)
+    // The clock is what a card holds under the loop's power; cards differ by some 6%.
     // Measured (MI355X, medians of alternating runs in one process, us; "one stage"
     // is the form with both operands of the next K block fetched at the step's
     // start and drained at its end):
@@ -516,7 +517,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     //   grouped variable K, 2048x7168      1238.2      1203.4      1143.7
     //   MX 8192 x 28672 x 8192             1445.4      1392.7      1365.0
     // (before the skip of the DMAs past the last block, worth another 0.5-1.5% to
-    // the ping-pong loop),
+    // the ping-pong loop); with few K blocks per tile, operands in the caches:
+    //   tensorwise 8192 x 8192 x 512         51.3        52.0
+    //   x 1024                               73.9        71.6
+    //   x 2048                              115.6       110.9
+    //   1x128 by 128x128, x 512              55.0        56.6
+    //   x 1024                               80.9        80.4
+    //   x 2048                              127.0       125.6
+    // (the last three on another card, before zero_acc below: 54.8 / 58.4 / 57.9, 80.0 /
+    // 80.6 / 81.1 and 126.2 / 126.5 / 130.2 for the interleaved loop),
     // so 1-D by 1-D scales and MX take the interleaved loop, the others ping-pong.
     // The accumulators' zeros, written while the first items are on their way: the
     // compiler puts these 128 VALU instructions per wave behind the wait (8192 x 8192 x
