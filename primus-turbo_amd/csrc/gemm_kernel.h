@@ -527,25 +527,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     // (the last three on another card, before zero_acc below: 54.8 / 58.4 / 57.9, 80.0 /
     // 80.6 / 81.1 and 126.2 / 126.5 / 130.2 for the interleaved loop),
     // so 1-D by 1-D scales and MX take the interleaved loop, the others ping-pong.
-    // The accumulators' zeros, written while the first items are on their way: the
-    // compiler puts these 128 VALU instructions per wave behind the wait (8192 x 8192 x
-    // 512, four tiles per CU: tensorwise 53.9 -> 52.0 us, 1x128 by 128x128 55.4 -> 53.5).
-    auto zero_acc = [&] {
-#pragma unroll
-        for (int j = 0; j < TN_; ++j)
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                // element by element: as one 4-register operand the accumulators' FMAs
-                // in the loop take their 8-byte form (1.5% slower)
-                float x[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    x[r] = 0.0f;
-                    asm volatile("" : "+v"(x[r]));
-                }
-                acc[j][i] = v4f{x[0], x[1], x[2], x[3]};
-            }
-    };
     // a phase's barrier: this wave's LDS reads are back, and all but its newest 8
     // item DMAs (and one of scales) have landed; all of them where the items that
     // would follow (of K block kb) do not exist
@@ -573,7 +554,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
             };
             issue(0, 0); issue(0, 2); issue(0, 1); issue(0, 3);
             issue(1, 0); issue(1, 2); issue(1, 1);
-            zero_acc();
             wait_items(1);
             const bool late = wave >= 4;
             if (late) asm volatile("s_barrier" ::: "memory");
@@ -696,7 +676,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
                 }
             };
             issue(0, 0); issue(0, 2); issue(0, 1); issue(0, 3);
-            zero_acc();
             // block 0's scales, a0, a1 and b0 have landed (requesting block 1 behind this
             // wait instead of ahead of it: 66.8 -> 64.7 us at 7168 x 2048 x 4096)
             asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
