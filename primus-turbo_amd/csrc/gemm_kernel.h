@@ -502,8 +502,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     // the clock second.  Busy share and clock on one card, at 4096 x 18432 x 7168 (1-D
     // by 1-D: 18432 x 7168 x 4096), and those of a loop of the same MFMAs and VALU
     // instructions on registers alone:
-    //   tensorwise 77% at 1.69 GHz (99% at 2.01)     1x128 by 128x128 60% at 1.86 (98% at 1.78)
-    //   1x128 by 1x128 45% at 2.07 (72% at 1.97)     MX 65% at 1.89 (99% at 2.05)
+    //   tensorwise 76% at 1.74 GHz (99% at 2.07)     1x128 by 128x128 61% at 1.89 (98% at 1.86)
+    //   1x128 by 1x128 45% at 2.16 (72% at 2.05)     MX 65% at 1.99 (99% at 2.14)
     // The clock is what a card holds under the loop's power; cards differ by some 6%.
     // Measured (MI355X, medians of alternating runs in one process, us; "one stage"
     // is the form with both operands of the next K block fetched at the step's
@@ -518,14 +518,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g, const int64_t bid) 
     //   MX 8192 x 28672 x 8192             1445.4      1392.7      1365.0
     // (before the skip of the DMAs past the last block, worth another 0.5-1.5% to
     // the ping-pong loop); with few K blocks per tile, operands in the caches:
-    //   tensorwise 8192 x 8192 x 512         51.3        52.0
-    //   x 1024                               73.9        71.6
-    //   x 2048                              115.6       110.9
-    //   1x128 by 128x128, x 512              55.0        56.6
-    //   x 1024                               80.9        80.4
-    //   x 2048                              127.0       125.6
-    // (the last three on another card, before zero_acc below: 54.8 / 58.4 / 57.9, 80.0 /
-    // 80.6 / 81.1 and 126.2 / 126.5 / 130.2 for the interleaved loop),
+    //   tensorwise 8192 x 8192 x 512         51.9        54.2
+    //   x 1024                               74.9        73.2
+    //   x 2048                              115.8       112.7
+    //   1x128 by 128x128, x 512              54.6        57.7        57.2
+    //   x 1024                               81.1        81.6        81.0
+    //   x 2048                              126.7       126.5       130.1
+    // (the interleaved column of these rows on another card, where ping-pong took 57.7,
+    // 80.7 and 126.1),
     // so 1-D by 1-D scales and MX take the interleaved loop, the others ping-pong.
     // a phase's barrier: this wave's LDS reads are back, and all but its newest 8
     // item DMAs (and one of scales) have landed; all of them where the items that
